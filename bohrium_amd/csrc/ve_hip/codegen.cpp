@@ -509,7 +509,10 @@ void Writer::collect() {
             always_array.insert(i->operand[0].base);
             index_checked.insert(i->operand[0].base);
         }
-        if (i->has_constant()) const_instrs.push_back(i);
+        // (a sweep's constant is its axis: it shapes the loops and is no argument.  The fuser rewrites it
+        // when it swaps axes, so shared with an equal constant it would be re-read from the flush as the
+        // axis that the program named.)
+        if (i->has_constant() && !bh_opcode_is_sweep(i->opcode)) const_instrs.push_back(i);
     }
     for (const bh_base *b : unit.getAllFrees()) {
         if (!bid.count(b)) {
@@ -712,7 +715,7 @@ void Writer::emit_instr(const bh_instruction &instr, Scope &sc, int ind) {
         for (size_t o = 0; o < instr.operand.size(); ++o) {
             const bh_view &v = instr.operand[o];
             if (v.isConstant()) {
-                ops.push_back(const_ref(instr));
+                ops.push_back(bh_opcode_is_sweep(instr.opcode) ? std::string() : const_ref(instr));
             } else if (o == 0 && bh_opcode_is_reduction(instr.opcode) && instr.operand[1].ndim > 1) {
                 ops.push_back(ref(sc, v, instr.sweep_axis()));
             } else {

@@ -290,3 +290,33 @@ def test_persistent_plan_covers_every_launch_in_dependency_order(tmp_path):
     assert len(gather_plans) == 40
     for i in gather_plans:
         assert min(level_of(t) for t, _, _ in mains[i]) > last_map_level
+
+
+AXIS_CONSTANT_DRIVER = r"""
+import sys
+sys.path.insert(0, %(root)r)
+import numpy as np, bohrium_amd as bh
+y = bh.empty((70, 9), np.int64)
+bh.flush()
+def program():
+    x = y %% 97
+    return [x.sum(axis=0), (x * x + 1).max(axis=0)]
+r = program()
+bh.flush()
+"""
+
+
+def test_an_axis_is_no_argument(tmp_path):
+    """The axis of a swapped reduction (0 in the program, 1 in the loop nest) shares no kernel argument with the
+    constant 1 of the same kernel: the argument was read from the program's axis, so x + 1 added 0."""
+    env = dict(os.environ, BH_HIP_DRY_RUN="1", BH_HIP_DUMP_DIR=str(tmp_path))
+    r = subprocess.run([sys.executable, "-c", AXIS_CONSTANT_DRIVER % {"root": ROOT}], env=env, stdout=subprocess.PIPE,
+                       stderr=subprocess.STDOUT, text=True, timeout=600)
+    assert r.returncode == 0, r.stdout[-3000:]
+    values = []
+    for f in os.listdir(str(tmp_path)):
+        for line in open(os.path.join(str(tmp_path), f)):
+            w = line.split()
+            if w[:1] == ["param"] and w[1] == "int64_t" and w[2][0] == "c" and w[3] == "bytes":
+                values.append(int.from_bytes(bytes(int(b) for b in w[4:]), "little", signed=True))
+    assert sorted(v for v in values if 0 < v < 100) == [1, 97], values  # the program's +1 and % 97
