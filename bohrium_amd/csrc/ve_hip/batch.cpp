@@ -342,7 +342,8 @@ void EngineHip::buildSchedule(CachedFlush &cf) {
     if (batch_min <= 0) return;
     std::unordered_map<uint64_t, size_t> count;
     for (const CachedKernel &ck : cf.kernels)
-        for (const KernelPlan &p : ck.plans) ++count[p.source_hash];
+        for (const KernelPlan &p : ck.plans)
+            if (p.strategy != Strategy::SEG_REDUCE) ++count[p.source_hash];
     bool any = false;
     for (const auto &kv : count) any |= kv.second >= static_cast<size_t>(batch_min);
     if (!any) return;
@@ -393,7 +394,10 @@ void EngineHip::buildSchedule(CachedFlush &cf) {
         Level &lv = sched->levels[L];
         for (uint64_t h : hash_order[L]) {
             std::vector<PlanRef> &items = by_hash[L][h];
-            if (items.size() >= static_cast<size_t>(batch_min)) {
+            // (a segmented reduction fills the chip by itself and finalizes with a grid of its own)
+            const bool batchable =
+                cf.kernels[items[0].kernel].plans[items[0].plan].strategy != Strategy::SEG_REDUCE;
+            if (batchable && items.size() >= static_cast<size_t>(batch_min)) {
                 sched->groups.emplace_back(new BatchGroup());
                 sched->groups.back()->items = std::move(items);
                 lv.groups.push_back(sched->groups.size() - 1);

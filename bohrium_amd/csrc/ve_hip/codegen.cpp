@@ -23,6 +23,7 @@ const char *strategy_name(Strategy s) {
         case Strategy::SCAN: return "scan";
         case Strategy::SERIAL: return "serial";
         case Strategy::ROW_REDUCE: return "row";
+        case Strategy::SEG_REDUCE: return "seg";
     }
     return "?";
 }
@@ -377,8 +378,13 @@ private:
     const bh_instruction *scan_instr = nullptr;
     std::string scan_sink;
 
+    /* Launch-shape arguments of a skeleton (plan-time values passed as kernel arguments, so that the
+     * source does not depend on the sizes). */
+    std::vector<std::pair<std::string, int64_t> > shape_args;
+
     std::ostringstream body;
-    std::string main_body;  // FULL_REDUCE: the main kernel's body while `body` holds the finalize's
+    // FULL_REDUCE, SEG_REDUCE: the main kernel's body while `body` holds the finalize's
+    std::string main_body;
 
     void collect();
     int view_id(const bh_view &v) {
@@ -484,6 +490,7 @@ private:
     std::vector<const bh_view *> preloadable(const LoopB &l);
     void emit_map();
     void emit_row_reduce();
+    void emit_seg_reduce();
     void emit_full_reduce();
     void emit_scan();
     void emit_serial();
@@ -761,6 +768,7 @@ std::vector<KernelParam> Writer::parameters() {
         const int64_t n = b->nelem();
         lit("int64_t", "nb" + std::to_string(bid.at(b)), &n, 8, 8);
     }
+    for (const auto &a : shape_args) lit("int64_t", a.first, &a.second, 8, 8);
     for (size_t j = 0; j < const_params.size(); ++j) {
         const bh_constant &c = const_params[j]->constant;
         const std::string cn = "c" + std::to_string(j);
@@ -1105,6 +1113,470 @@ void Writer::emit_row_reduce() {
     body << "  }\n";
     write_back(unit, ksc, 1);
     kp.grid = std::max<uint64_t>(1, std::min<uint64_t>((rows + 3) / 4, cfg.max_grid));
+}
+
+
+/* A segmented reduction: the innermost leading parallel loop P holds constant seeds of the reductions of
+ * one innermost loop C, C, and element-wise instructions after it.  C's sweeps reduce its own, last
+ * axis; C reads no reduction output, gathers and scatters nothing, and touches a base that it writes
+ * only through the written view (elements of one output may be computed by several threads). */
+struct SegForm {
+    const LoopB *C = nullptr;
+    std::vector<const bh_instruction *> seeds;
+    std::vector<InstrPtr> post;
+    std::set<const bh_base *> loop_temps;  // temporaries of P that only C uses
+    bool columns = false;  // the contiguous axis is P's (reduce over rows), else C's
+    int width = 1;         // elements of the contiguous axis that 16 bytes of the widest such view hold
+};
+
+// Shapes below this many elements keep the row and map skeletons (one small launch, batchable).
+constexpr uint64_t kSegMinItems = 1u << 16;
+
+SegForm seg_form(const LoopB &l0, const std::set<const bh_base *> &params) {
+    SegForm none, f;
+    const uint64_t p = std::max<uint64_t>(1, jitk::parallel_ranks(l0).first);
+    const std::vector<const LoopB *> chain = jitk::get_first_loop_blocks(l0);
+    if (chain.size() < p) return none;
+    const LoopB &P = *chain[p - 1];
+    std::vector<InstrPtr> before;
+    for (const Block &b : P._block_list) {
+        if (!b.isInstr()) {
+            if (f.C != nullptr) return none;
+            f.C = &b.getLoop();
+            continue;
+        }
+        const InstrPtr &i = b.getInstr();
+        if (bh_opcode_is_system(i->opcode)) continue;
+        if (bh_opcode_is_sweep(i->opcode) || i->opcode == BH_GATHER || i->opcode == BH_SCATTER ||
+            i->opcode == BH_COND_SCATTER || i->opcode == BH_RANDOM || i->opcode == BH_RANGE)
+            return none;
+        (f.C == nullptr ? before : f.post).push_back(i);
+    }
+    if (f.C == nullptr || !f.C->isInnermost() || f.C->_sweeps.empty() || f.C->size < 16) return none;
+    uint64_t outs_n = 1;
+    for (uint64_t r = 0; r < p; ++r) outs_n *= static_cast<uint64_t>(std::max<int64_t>(0, chain[r]->size));
+    if (outs_n * static_cast<uint64_t>(f.C->size) < kSegMinItems || outs_n >= (1ull << 31)) return none;
+    std::map<const bh_base *, const bh_view *> outs;
+    for (const InstrPtr &sw : f.C->_sweeps) {
+        if (!bh_opcode_is_reduction(sw->opcode) || sw->sweep_axis() != f.C->rank ||
+            sw->sweep_axis() != sw->operand[1].ndim - 1 || outs.count(sw->operand[0].base))
+            return none;
+        outs[sw->operand[0].base] = &sw->operand[0];
+    }
+    for (const InstrPtr &i : before) {
+        if (i->opcode != BH_IDENTITY || !i->operand[1].isConstant()) return none;
+        auto o = outs.find(i->operand[0].base);
+        if (o == outs.end() || !(i->operand[0] == *o->second)) return none;
+        f.seeds.push_back(i.get());
+    }
+    // Every sweep output is seeded here (the partials start at the identity themselves).
+    for (const auto &o : outs) {
+        bool seeded = false;
+        for (const bh_instruction *i : f.seeds) seeded |= i->operand[0].base == o.first;
+        if (!seeded) return none;
+    }
+    std::map<const bh_base *, const bh_view *> written;
+    const std::vector<InstrPtr> body = jitk::allInstr(*f.C);
+    for (const InstrPtr &i : body) {
+        if (bh_opcode_is_system(i->opcode)) continue;
+        if (i->opcode == BH_GATHER || i->opcode == BH_SCATTER || i->opcode == BH_COND_SCATTER) return none;
+        if (i->operand[0].isConstant()) return none;
+        if (outs.count(i->operand[0].base)) {
+            if (!f.C->_sweeps.count(i)) return none;
+            continue;
+        }
+        auto w = written.find(i->operand[0].base);
+        if (w != written.end() && !(*w->second == i->operand[0])) return none;
+        written[i->operand[0].base] = &i->operand[0];
+    }
+    for (const InstrPtr &i : body)
+        for (size_t o = 0; o < i->operand.size(); ++o) {
+            const bh_view &v = i->operand[o];
+            if (v.isConstant()) continue;
+            if (v.hasSlide()) return none;
+            auto w = written.find(v.base);
+            if (w != written.end() && !(v == *w->second)) return none;
+            if (o > 0 && outs.count(v.base)) return none;
+        }
+    for (const InstrPtr &i : f.post)
+        for (size_t o = 0; o < i->operand.size(); ++o) {
+            const bh_view &v = i->operand[o];
+            if (v.isConstant()) continue;
+            if (v.hasSlide()) return none;
+            // (an element that C wrote may still be on its way from another lane)
+            if (written.count(v.base)) return none;
+            auto r = outs.find(v.base);
+            if (r != outs.end() && (o == 0 || !(v == *r->second))) return none;
+        }
+    // Temporaries of the parallel loops other than the sweep outputs: the reduction loop's own when
+    // nothing outside it touches them (a lifted free), else the block has another form.
+    const std::set<bh_base *> c_temps = f.C->getLocalTemps();
+    for (uint64_t r = 0; r < p; ++r)
+        for (bh_base *b : chain[r]->getLocalTemps()) {
+            if (outs.count(b) || c_temps.count(b)) continue;
+            bool in_body = false, in_post = false;
+            for (const InstrPtr &i : body)
+                for (const bh_view &v : i->operand) in_body |= !v.isConstant() && v.base == b;
+            for (const InstrPtr &i : f.post)
+                for (const bh_view &v : i->operand) in_post |= !v.isConstant() && v.base == b;
+            if (in_body && in_post) return none;
+            if (in_body) f.loop_temps.insert(b);
+        }
+    // The contiguous axis of the arrays that C reads, weighted by their element size.
+    int64_t cols = 0, rows = 0;
+    int widest = 1;
+    std::set<VKey> seen;
+    const int64_t a = static_cast<int64_t>(p) - 1, c = f.C->rank;
+    for (const InstrPtr &i : body)
+        for (size_t o = 1; o < i->operand.size(); ++o) {
+            const bh_view &v = i->operand[o];
+            if (v.isConstant() || !params.count(v.base) || v.ndim <= c || !seen.insert(vkey(v)).second) continue;
+            const int sz = bh_type_size(v.base->dtype());
+            if (v.stride[c] == 1 && v.shape[c] > 1 && v.stride[a] != 1) {
+                rows += sz;
+                widest = std::max(widest, sz);
+            } else if (v.stride[a] == 1 && v.shape[a] > 1 && v.stride[c] != 1) {
+                cols += sz;
+                widest = std::max(widest, sz);
+            }
+        }
+    if (rows == cols) return none;
+    f.columns = cols > rows;
+    f.width = std::max(1, std::min(4, 16 / widest));
+    return f;
+}
+
+// ---- SEG_REDUCE
+// Bound by HBM when the whole chip loads.  What the row skeleton left idle: a column sum ran one wave
+// per column with its lanes a row apart (one 64-byte request per lane and element), and few outputs
+// gave few waves.  Here lanes always run along the contiguous axis with 16-byte loads, and the reduced
+// axis is cut into `splits` pieces until the launch has about kSegBlocks workgroups.  Measured on float32:
+// mean, variance and standardised matrix of 100000 x 500 by columns 1792 -> 231 us (the two reduction
+// kernels 0.81 and 0.88 ms before), of 16384 x 3000 by rows 223 -> 198 us (4-byte loads before).
+constexpr uint64_t kSegBlocks = 2048;
+
+void Writer::emit_seg_reduce() {
+    const LoopB &l0 = unit._block_list.back().getLoop();
+    const uint64_t p = std::max<uint64_t>(1, jitk::parallel_ranks(l0).first);
+    const std::vector<const LoopB *> chain = jitk::get_first_loop_blocks(l0);
+    const SegForm f = seg_form(l0, std::set<const bh_base *>(kp.params.begin(), kp.params.end()));
+    if (f.C == nullptr) throw std::logic_error("seg skeleton: block has another form");
+    for (const bh_instruction *i : f.seeds) skip.insert(i);
+    const LoopB &C = *f.C, &P = *chain[p - 1];
+    uint64_t outs_n = 1;
+    for (uint64_t r = 0; r < p; ++r) outs_n *= static_cast<uint64_t>(chain[r]->size);
+    const uint64_t R = static_cast<uint64_t>(C.size);
+    kp.work_items = outs_n * R;
+    const uint64_t W = kp.block;
+    const std::string rk = std::to_string(C.rank), pk = std::to_string(p - 1);
+    const std::string nR = "n" + std::to_string(lid.at(&C));
+
+    // Vector width, threads along the outputs / lanes per row, splits of the reduced axis.
+    int V = f.width;
+    const int U = f.columns ? (V >= 4 ? 4 : 8) : 4;
+    uint64_t lanes = 1, row_blocks = 1, splits = 1, chunk = R, w = 1;
+    if (f.columns) {
+        while (P.size % V != 0) V /= 2;  // a thread's outputs are V neighbours of one innermost row
+        const uint64_t groups = outs_n / static_cast<uint64_t>(V);
+        row_blocks = (groups + W - 1) / W;
+        w = (groups + row_blocks - 1) / row_blocks;
+        const uint64_t ty = W / w;
+        const uint64_t step = ty * static_cast<uint64_t>(U);
+        splits = std::max<uint64_t>(1, std::min((kSegBlocks + row_blocks - 1) / row_blocks, R / (2 * step)));
+        chunk = (R + splits - 1) / splits;
+        splits = (R + chunk - 1) / chunk;
+    } else {
+        // A workgroup per row for long rows (and for moderate ones when there are few), else a wave, and
+        // fewer lanes for short rows: each lane loads at least twice.
+        const uint64_t wide = W * static_cast<uint64_t>(2 * V);
+        lanes = R >= wide * static_cast<uint64_t>(U) || (outs_n < kSegBlocks && R >= wide) ? W : 64;
+        while (lanes > 4 && lanes <= 64 && lanes * static_cast<uint64_t>(2 * V) > R) lanes /= 2;
+        const uint64_t per_block = W / lanes;
+        row_blocks = (outs_n + per_block - 1) / per_block;
+        const uint64_t step = lanes * static_cast<uint64_t>(V * U);
+        if (lanes == 256)
+            splits = std::max<uint64_t>(1, std::min((kSegBlocks + row_blocks - 1) / row_blocks, R / (2 * step)));
+        chunk = (R + splits - 1) / splits;
+        chunk = (chunk + lanes * V - 1) / (lanes * V) * (lanes * V);
+        splits = (R + chunk - 1) / chunk;
+    }
+    const bool split = splits > 1;
+    kp.grid = row_blocks * splits;
+    shape_args = {{"sg_nb", static_cast<int64_t>(row_blocks)}, {"sg_ch", static_cast<int64_t>(chunk)}};
+    if (f.columns) shape_args.emplace_back("sg_w", static_cast<int64_t>(w));
+
+    struct Acc {
+        InstrPtr instr;
+        bh_type t;
+        std::string T, var, ident;
+    };
+    std::vector<Acc> accs;
+    std::vector<InstrPtr> sweeps(C._sweeps.begin(), C._sweeps.end());
+    std::sort(sweeps.begin(), sweeps.end(), [](const InstrPtr &x, const InstrPtr &y) { return x->origin_id < y->origin_id; });
+    for (const InstrPtr &s : sweeps) {
+        Acc a;
+        a.instr = s;
+        a.t = s->operand[0].base->dtype();
+        a.T = hip_type(a.t);
+        a.var = "q" + std::to_string(accs.size());
+        a.ident = literal(jitk::sweep_identity(s->opcode, a.t));
+        accs.push_back(a);
+    }
+    auto op_lambda = [&](const Acc &a) {
+        return "auto op_ = [](" + a.T + " x, " + a.T + " y) -> " + a.T + " { return " +
+               combine_expr(a.instr->opcode, "x", "y") + "; };";
+    };
+    // Partials: per accumulator a slab of splits x outputs.
+    uint64_t scratch = 0;
+    if (split) {
+        for (size_t k = 0; k < accs.size(); ++k) {
+            shape_args.emplace_back("sg_o" + std::to_string(k), static_cast<int64_t>(scratch));
+            scratch += (splits * outs_n * static_cast<uint64_t>(bh_type_size(accs[k].t)) + 255) / 256 * 256;
+        }
+        kp.scratch_bytes = static_cast<int64_t>(scratch);
+    }
+    std::string outs_expr = "1";
+    for (uint64_t r = 0; r < p; ++r) outs_expr += " * n" + std::to_string(lid.at(chain[r]));
+    Scope ksc;
+    // i0 .. i{p-1} of the flat output number `e` (32-bit: there are fewer than 2^31 outputs)
+    auto decode = [&](int ind, const std::string &e) {
+        const std::string pad(2 * ind, ' ');
+        body << pad << "uint32_t d_ = (uint32_t)(" << e << ");\n";
+        for (int64_t r = static_cast<int64_t>(p) - 1; r >= 1; --r)
+            body << pad << "const int64_t i" << r << " = (int64_t)(d_ % (uint32_t)n" << lid.at(chain[r])
+                 << "); d_ /= (uint32_t)n" << lid.at(chain[r]) << ";\n";
+        body << pad << "const int64_t i0 = (int64_t)d_;\n";
+    };
+    // The rest of one output: its reductions are in accumulator registers `var(k)`.
+    auto finish = [&](int ind, const std::function<std::string(size_t)> &var) {
+        std::vector<Scope> scopes(p);
+        const Scope *parent = &ksc;
+        for (uint64_t r = 0; r < p; ++r) {
+            scopes[r].parent = parent;
+            indent(body, ind + static_cast<int>(r));
+            body << "{\n";
+            declare_scope(*chain[r], scopes[r], ind + 1 + static_cast<int>(r));
+            parent = &scopes[r];
+        }
+        const int in = ind + static_cast<int>(p);
+        Scope &ps = scopes[p - 1];
+        for (size_t k = 0; k < accs.size(); ++k) {
+            const bh_instruction &s = *accs[k].instr;
+            indent(body, in);
+            body << ref(ps, s.operand[0], static_cast<int>(s.sweep_axis())) << " = " << var(k) << ";\n";
+        }
+        for (const InstrPtr &i : f.post) emit_instr(*i, ps, in);
+        for (int64_t r = static_cast<int64_t>(p) - 1; r >= 0; --r) {
+            write_back(*chain[r], scopes[r], ind + 1 + static_cast<int>(r));
+            indent(body, ind + static_cast<int>(r));
+            body << "}\n";
+        }
+    };
+    // One element of C in a scope whose accumulators are var(k); `pre` names preloaded inputs.
+    auto element = [&](int ind, const Scope *pre, const std::function<std::string(size_t)> &var) {
+        Scope al;
+        al.parent = pre;
+        for (size_t k = 0; k < accs.size(); ++k) al.alias[accs[k].instr->operand[0].base] = var(k);
+        Scope sc;
+        sc.parent = &al;
+        for (const bh_base *b : f.loop_temps) {
+            sc.tmps.insert(b);
+            indent(body, ind);
+            body << hip_type(b->dtype()) << " t" << bid.at(b) << ";\n";
+        }
+        declare_scope(C, sc, ind);
+        emit_blocks(C, sc, ind);
+        write_back(C, sc, ind);
+    };
+    const std::vector<const bh_view *> reads = preloadable(C);
+    // `U` x `V` elements: load every read-only input, then compute.  head(u, v) declares the indices.
+    auto group = [&](int ind, int nu, int nv, const std::function<void(int, int, int)> &head,
+                     const std::function<std::string(size_t, int)> &var) {
+        const std::string pad(2 * ind, ' ');
+        auto ld = [&](size_t k, int u, int v) {
+            return "ld" + std::to_string(k) + "_" + std::to_string(u) + "_" + std::to_string(v);
+        };
+        for (int u = 0; u < nu; ++u)
+            for (int v = 0; v < nv; ++v)
+                for (size_t k = 0; k < reads.size(); ++k)
+                    body << pad << hip_type(reads[k]->base->dtype()) << " " << ld(k, u, v) << ";\n";
+        for (int u = 0; u < nu; ++u)
+            for (int v = 0; v < nv; ++v) {
+                if (reads.empty()) break;
+                body << pad << "{\n";
+                head(ind + 1, u, v);
+                for (size_t k = 0; k < reads.size(); ++k)
+                    body << pad << "  " << ld(k, u, v) << " = " << ref(ksc, *reads[k]) << ";\n";
+                body << pad << "}\n";
+            }
+        for (int u = 0; u < nu; ++u)
+            for (int v = 0; v < nv; ++v) {
+                Scope pre;
+                pre.parent = &ksc;
+                for (size_t k = 0; k < reads.size(); ++k) pre.preload[vkey(*reads[k])] = ld(k, u, v);
+                body << pad << "{\n";
+                head(ind + 1, u, v);
+                element(ind + 1, &pre, [&](size_t k) { return var(k, v); });
+                body << pad << "}\n";
+            }
+    };
+    auto store_partial = [&](size_t k, const std::string &out, const std::string &value) {
+        return "((" + accs[k].T + " *)(bh_scratch + sg_o" + std::to_string(k) + "))[sp_ * outs_ + " + out + "] = " + value + ";\n";
+    };
+
+    body << "  const int64_t outs_ = " << outs_expr << ";\n";
+    body << "  const int64_t sp_ = bh_bid / (unsigned)sg_nb, cb_ = bh_bid % (unsigned)sg_nb;\n";
+    body << "  const int64_t r0_ = sp_ * sg_ch, r1_ = r0_ + sg_ch < " << nR << " ? r0_ + sg_ch : " << nR << ";\n";
+    const std::string sV = std::to_string(V);
+    if (f.columns) {
+        // Thread (tx_, ty_): outputs [e_, e_ + V), rows r0_ + ty_, + ty step, ...
+        body << "  const unsigned w_ = (unsigned)sg_w, tys_ = BH_WG / w_;\n";
+        body << "  const unsigned ty_ = threadIdx.x / w_, tx_ = threadIdx.x - ty_ * w_;\n";
+        body << "  const int64_t e_ = (cb_ * w_ + tx_) * " << V << ";\n";
+        body << "  const bool on_ = ty_ < tys_ && e_ < outs_;\n";
+        for (size_t k = 0; k < accs.size(); ++k)
+            for (int v = 0; v < V; ++v)
+                body << "  " << accs[k].T << " " << accs[k].var << "_" << v << " = " << accs[k].ident << ";\n";
+        auto var = [&](size_t k, int v) { return accs[k].var + "_" + std::to_string(v); };
+        body << "  if (on_) {\n";
+        // (the first output's indices; the innermost one advances by v)
+        {
+            const std::string inner = "i" + pk;
+            body << "    uint32_t d_ = (uint32_t)e_;\n";
+            for (int64_t r = static_cast<int64_t>(p) - 1; r >= 1; --r)
+                body << "    const int64_t b" << r << "_ = (int64_t)(d_ % (uint32_t)n" << lid.at(chain[r])
+                     << "); d_ /= (uint32_t)n" << lid.at(chain[r]) << ";\n";
+            body << "    const int64_t b0_ = (int64_t)d_;\n";
+            for (int64_t r = 0; r + 1 < static_cast<int64_t>(p); ++r)
+                body << "    const int64_t i" << r << " = b" << r << "_;\n";
+            auto head = [&](int ind, int u, int v) {
+                indent(body, ind);
+                body << "const int64_t " << inner << " = b" << pk << "_ + " << v << ", i" << rk << " = r_ + " << u
+                     << " * (int64_t)tys_;\n";
+            };
+            body << "    int64_t r_ = r0_ + ty_;\n";
+            body << "    for (; r_ + " << U - 1 << " * (int64_t)tys_ < r1_; r_ += " << U << " * (int64_t)tys_) {\n";
+            group(3, U, V, head, var);
+            body << "    }\n";
+            body << "    for (; r_ < r1_; r_ += tys_) {\n";
+            group(3, 1, V, head, var);
+            body << "    }\n";
+        }
+        body << "  }\n";
+        // Fold the rows of the workgroup through LDS, in row order.
+        int largest = 1;
+        for (const Acc &a : accs) largest = std::max(largest, bh_type_size(a.t));
+        body << "  __shared__ __attribute__((aligned(16))) unsigned char bh_lds_[BH_WG * " << V * largest << "];\n";
+        for (size_t k = 0; k < accs.size(); ++k) {
+            const Acc &a = accs[k];
+            body << "  { " << op_lambda(a) << "\n";
+            body << "    " << a.T << " *l_ = (" << a.T << " *)bh_lds_;\n";
+            if (k > 0) body << "    __syncthreads();\n";
+            body << "    if (on_) {\n";
+            for (int v = 0; v < V; ++v) body << "      l_[threadIdx.x * " << V << " + " << v << "] = " << var(k, v) << ";\n";
+            body << "    }\n    __syncthreads();\n";
+            body << "    if (on_ && ty_ == 0) {\n      for (unsigned t_ = 1; t_ < tys_; ++t_) {\n";
+            for (int v = 0; v < V; ++v)
+                body << "        " << var(k, v) << " = op_(" << var(k, v) << ", l_[(t_ * w_ + tx_) * " << V << " + " << v << "]);\n";
+            body << "      }\n    }\n  }\n";
+        }
+        body << "  if (!on_ || ty_ != 0) return;\n";
+        for (int v = 0; v < V; ++v) {
+            if (split) {
+                for (size_t k = 0; k < accs.size(); ++k)
+                    body << "  " << store_partial(k, "e_ + " + std::to_string(v), var(k, v));
+            } else {
+                body << "  {\n";
+                decode(2, "e_ + " + std::to_string(v));
+                finish(2, [&](size_t k) { return var(k, v); });
+                body << "  }\n";
+            }
+        }
+    } else {
+        // `lanes` threads per output, V neighbouring elements each.
+        const std::string G = std::to_string(lanes);
+        body << "  const unsigned l_ = threadIdx.x % " << G << "u;\n";
+        body << "  const int64_t e_ = cb_ * " << W / lanes << " + threadIdx.x / " << G << "u;\n";
+        body << "  const bool on_ = e_ < outs_;\n";
+        for (const Acc &a : accs) body << "  " << a.T << " " << a.var << " = " << a.ident << ";\n";
+        auto var = [&](size_t k, int) { return accs[k].var; };
+        body << "  if (on_) {\n";
+        decode(2, "e_");
+        auto head = [&](int ind, int u, int v) {
+            indent(body, ind);
+            body << "const int64_t i" << rk << " = r_ + " << u * static_cast<int64_t>(lanes) * V + v << ";\n";
+        };
+        body << "    int64_t r_ = r0_ + (int64_t)l_ * " << V << ";\n";
+        body << "    for (; r_ + " << (U - 1) * static_cast<int64_t>(lanes) * V + V << " <= r1_; r_ += " << U * static_cast<int64_t>(lanes) * V << ") {\n";
+        group(3, U, V, head, var);
+        body << "    }\n";
+        body << "    for (; r_ + " << V << " <= r1_; r_ += " << static_cast<int64_t>(lanes) * V << ") {\n";
+        group(3, 1, V, head, var);
+        body << "    }\n";
+        if (V > 1) {
+            // the last (r1_ - r0_) mod V elements, one lane each
+            body << "    r_ = r1_ - (r1_ - r0_) % " << V << " + l_;\n    if (r_ < r1_) {\n";
+            group(3, 1, 1, head, var);
+            body << "    }\n";
+        }
+        body << "  }\n";
+        if (lanes == 256)
+            body << "  __shared__ __attribute__((aligned(16))) unsigned char bh_lds_[BH_WAVES * 16];\n";
+        for (const Acc &a : accs) {
+            body << "  { " << op_lambda(a) << "\n    " << a.var << " = ";
+            if (lanes == 256) {
+                body << "bh_block_reduce(" << a.var << ", op_, (" << a.T << " *)bh_lds_);\n    __syncthreads(); }\n";
+            } else {
+                body << "bh_group_reduce<" << G << ">(" << a.var << ", op_); }\n";
+            }
+        }
+        body << "  if (!on_ || l_ != 0) return;\n";
+        if (split) {
+            for (size_t k = 0; k < accs.size(); ++k) body << "  " << store_partial(k, "e_", accs[k].var);
+        } else {
+            body << "  {\n";
+            decode(2, "e_");
+            finish(2, [&](size_t k) { return accs[k].var; });
+            body << "  }\n";
+        }
+    }
+    if (!split) return;
+    main_body = body.str();
+    body.str("");
+    body.clear();
+
+    // Finalize: 16 outputs x 16 slices of the partials per workgroup, folded in split order within a
+    // slice and then across slices; the first slice's thread finishes the output.
+    shape_args.emplace_back("sg_ns", static_cast<int64_t>(splits));
+    kp.fin_name = "bh_kernel_fin";
+    kp.fin_grid = (outs_n + 15) / 16;
+    body << "  const int64_t outs_ = " << outs_expr << ";\n";
+    body << "  const unsigned tx_ = threadIdx.x & 15u, ty_ = threadIdx.x >> 4;\n";
+    body << "  const int64_t e_ = (int64_t)bh_bid * 16 + tx_;\n";
+    body << "  const bool on_ = e_ < outs_;\n";
+    int largest = 1;
+    for (const Acc &a : accs) largest = std::max(largest, bh_type_size(a.t));
+    body << "  __shared__ __attribute__((aligned(16))) unsigned char bh_lds_[16 * 17 * " << largest << "];\n";
+    body << "  const int64_t ps_ = (sg_ns + 15) / 16, p0_ = ty_ * ps_, p1_ = p0_ + ps_ < sg_ns ? p0_ + ps_ : sg_ns;\n";
+    for (size_t k = 0; k < accs.size(); ++k) {
+        const Acc &a = accs[k];
+        body << "  " << a.T << " " << a.var << " = " << a.ident << ";\n";
+        body << "  { " << op_lambda(a) << "\n";
+        body << "    const " << a.T << " *s_ = (const " << a.T << " *)(bh_scratch + sg_o" << k << ");\n";
+        body << "    if (on_) {\n      int64_t j_ = p0_;\n";
+        body << "      for (; j_ + 8 <= p1_; j_ += 8) {\n        " << a.T << " x_[8];\n#pragma unroll\n"
+             << "        for (int u_ = 0; u_ < 8; ++u_) x_[u_] = s_[(j_ + u_) * outs_ + e_];\n#pragma unroll\n"
+             << "        for (int u_ = 0; u_ < 8; ++u_) " << a.var << " = op_(" << a.var << ", x_[u_]);\n      }\n";
+        body << "      for (; j_ < p1_; ++j_) " << a.var << " = op_(" << a.var << ", s_[j_ * outs_ + e_]);\n    }\n";
+        body << "    " << a.T << " *l_ = (" << a.T << " *)bh_lds_;\n";
+        if (k > 0) body << "    __syncthreads();\n";
+        body << "    l_[ty_ * 17 + tx_] = " << a.var << ";\n    __syncthreads();\n";
+        body << "    if (ty_ == 0)\n      for (int t_ = 1; t_ < 16; ++t_) " << a.var << " = op_(" << a.var << ", l_[t_ * 17 + tx_]);\n  }\n";
+    }
+    body << "  if (!on_ || ty_ != 0) return;\n  {\n";
+    decode(2, "e_");
+    finish(2, [&](size_t k) { return accs[k].var; });
+    body << "  }\n";
 }
 
 // ---- MAP: grid-stride over the flattened leading parallel ranks
@@ -1552,12 +2024,14 @@ KernelPlan Writer::plan(Strategy s) {
     switch (s) {
         case Strategy::MAP: emit_map(); break;
         case Strategy::ROW_REDUCE: emit_row_reduce(); break;
+        case Strategy::SEG_REDUCE: emit_seg_reduce(); break;
         case Strategy::FULL_REDUCE: emit_full_reduce(); break;
         case Strategy::SCAN: emit_scan(); break;
         case Strategy::SERIAL: emit_serial(); break;
     }
     std::vector<KernelParam> params = parameters();
-    if (s == Strategy::FULL_REDUCE || s == Strategy::SCAN) {
+    const bool two_kernels = !kp.fin_name.empty();
+    if (s == Strategy::FULL_REDUCE || s == Strategy::SCAN || (s == Strategy::SEG_REDUCE && two_kernels)) {
         params.push_back({"unsigned char *", "bh_scratch", true});
         ArgSpec a;
         a.kind = ArgSpec::SCRATCH_PTR;
@@ -1588,15 +2062,17 @@ KernelPlan Writer::plan(Strategy s) {
         nlist += (i ? ", " : "") + params[i].name;
     }
     std::ostringstream dev;
-    const std::string main_src = s == Strategy::FULL_REDUCE ? main_body : body.str();
+    const std::string main_src = two_kernels ? main_body : body.str();
     // Gathers mark an index outside its base in bh_bad_; the flag is raised once per thread at the end
     // (every early return in a body comes before its first gather).
     const std::string bad0 = kp.uses_gather_flag ? "  bool bh_bad_ = false;\n" : "";
     const std::string bad1 = kp.uses_gather_flag ? "  if (bh_bad_) atomicOr(bh_err, BH_ERR_INDEX);\n" : "";
     dev << "__device__ __forceinline__ void bh_main_(" << plist << (plist.empty() ? "" : ",\n    ")
         << "const unsigned bh_bid, const unsigned bh_nblk) {\n" << bad0 << main_src << bad1 << "}\n";
-    if (s == Strategy::FULL_REDUCE)
-        dev << "\n__device__ __forceinline__ void bh_fin_(" << plist << ") {\n" << bad0 << body.str() << bad1 << "}\n";
+    const bool seg = s == Strategy::SEG_REDUCE;
+    if (two_kernels)
+        dev << "\n__device__ __forceinline__ void bh_fin_(" << plist << (seg ? ",\n    const unsigned bh_bid" : "")
+            << ") {\n" << bad0 << body.str() << bad1 << "}\n";
     kp.device_code = dev.str();
     std::ostringstream src;
     // Occupancy hint for the main kernel (waves per SIMD the register allocator must allow).
@@ -1610,9 +2086,9 @@ KernelPlan Writer::plan(Strategy s) {
         << " " << kp.name << "("
         << plist << ") {\n  bh_main_(" << nlist << (nlist.empty() ? "" : ", ")
         << (remap ? "bh_xcd_block(blockIdx.x, gridDim.x)" : "blockIdx.x") << ", gridDim.x);\n}\n";
-    if (s == Strategy::FULL_REDUCE)
+    if (two_kernels)
         src << "\nextern \"C\" __global__ void __launch_bounds__(" << kp.block << ") " << kp.fin_name << "(" << plist
-            << ") {\n  bh_fin_(" << nlist << ");\n}\n";
+            << ") {\n  bh_fin_(" << nlist << (seg ? ", blockIdx.x" : "") << ");\n}\n";
     kp.source = src.str();
     return kp;
 }
@@ -1841,6 +2317,15 @@ std::string verify_kernel(const LoopB &kernel) {
     return err;
 }
 
+namespace {
+// The bases a unit addresses as arrays (its writer's parameters).
+std::set<const bh_base *> param_bases(const LoopB &unit) {
+    std::set<const bh_base *> out;
+    for (const bh_base *b : unit.getAllNonTemps()) out.insert(b);
+    return out;
+}
+} // namespace
+
 std::vector<KernelPlan> plan_kernel(const LoopB &kernel, const WriterConfig &cfg) {
     std::vector<KernelPlan> ret;
     auto emit = [&](LoopB unit, Strategy s) {
@@ -1887,7 +2372,14 @@ std::vector<KernelPlan> plan_kernel(const LoopB &kernel, const WriterConfig &cfg
         }
         LoopB unit(-1, 1, scalar_ids);
         unit._block_list.push_back(b);
-        if (s == Strategy::MAP && cfg.row_reduce && !row_lane_loops(l0).empty()) s = Strategy::ROW_REDUCE;
+        if (s == Strategy::MAP && cfg.row_reduce) {
+            unit.metadataUpdate();
+            if (seg_form(l0, param_bases(unit)).C != nullptr) {
+                s = Strategy::SEG_REDUCE;
+            } else if (!row_lane_loops(l0).empty()) {
+                s = Strategy::ROW_REDUCE;
+            }
+        }
         if (s == Strategy::FULL_REDUCE) {
             while (bi + 1 < blocks.size() && (blocks[bi + 1].isSystemOnly() || tail_block(blocks[bi + 1])))
                 unit._block_list.push_back(blocks[++bi]);

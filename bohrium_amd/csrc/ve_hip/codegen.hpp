@@ -13,6 +13,10 @@
  *   ROW_REDUCE   a map whose innermost parallel loop only seeds and reduces an inner
  *                loop (row sums of an expression): one wave per row, lanes stride the
  *                row (coalesced), wave64 butterfly, lane 0 stores.
+ *   SEG_REDUCE   one reduction loop per element of the parallel ranks (a sum over one axis of a
+ *                matrix) when the matrix is large: wide coalesced loads along whichever axis is
+ *                contiguous, and the reduced axis split over workgroups (partials folded by a
+ *                finalize kernel) when the outputs alone do not fill the chip.
  *   SERIAL       anything else, executed by one thread (always correct).
  * Per-opcode scalar semantics restate the reference's write_operation
  * (core/jitk/instruction.cpp:58-544) and engine.cpp:251-336 special forms.
@@ -28,7 +32,7 @@
 namespace bohrium {
 namespace vehip {
 
-enum class Strategy { MAP, FULL_REDUCE, SCAN, SERIAL, ROW_REDUCE };
+enum class Strategy { MAP, FULL_REDUCE, SCAN, SERIAL, ROW_REDUCE, SEG_REDUCE };
 const char *strategy_name(Strategy s);
 
 /* One kernel argument: either literal bytes known at plan time, or a pointer
@@ -58,9 +62,10 @@ struct KernelPlan {
     Strategy strategy = Strategy::SERIAL;
     std::string source;  // kernel source without the prelude
     std::string name;
-    /* FULL_REDUCE: a second kernel of the same module, launched with one workgroup right
-     * after `name` with the same arguments (folds the per-workgroup partials). */
+    /* FULL_REDUCE and split SEG_REDUCE: a second kernel of the same module, launched with fin_grid
+     * workgroups right after `name` with the same arguments (folds the per-workgroup partials). */
     std::string fin_name;
+    uint64_t fin_grid = 1;
     std::vector<ArgSpec> args;
     /* The body as device functions (bh_main_, and bh_fin_ for FULL_REDUCE) and their parameters,
      * one per ArgSpec: declaration, value type and name.  `source` adds the kernels calling them. */

@@ -413,7 +413,8 @@ void EngineHip::launchPlan(KernelPlan &plan, const std::vector<bh_base *> &ord2b
         t = std::chrono::steady_clock::now();
     }
     for (int o : plan.param_ordinals) ensureResident(ord2base[o]);
-    if (plan.strategy == Strategy::FULL_REDUCE) ensureScratch(reduce_scratch, reduce_scratch_bytes, plan.scratch_bytes, false);
+    if (plan.strategy == Strategy::FULL_REDUCE || plan.strategy == Strategy::SEG_REDUCE)
+        ensureScratch(reduce_scratch, reduce_scratch_bytes, plan.scratch_bytes, false);
     if (plan.strategy == Strategy::SCAN) ensureScratch(scan_scratch, scan_scratch_bytes, plan.scratch_bytes, true);
     uint8_t buf[4096];
     const size_t n = packArgs(plan, ord2base, instrs, plan.strategy == Strategy::SCAN ? scan_scratch : reduce_scratch,
@@ -430,9 +431,9 @@ void EngineHip::launchPlan(KernelPlan &plan, const std::vector<bh_base *> &ord2b
     errors_unchecked |= plan.uses_error_flag;
     if (recording != nullptr) recording->push_back({plan.function, plan.grid, plan.block, {buf, buf + n}});
     if (plan.fin_function != nullptr) {
-        check(bhhip_launch(plan.fin_function, 1, plan.block, buf, n), "kernel launch");
+        check(bhhip_launch(plan.fin_function, plan.fin_grid, plan.block, buf, n), "kernel launch");
         ++stats.launches;
-        if (recording != nullptr) recording->push_back({plan.fin_function, 1, plan.block, {buf, buf + n}});
+        if (recording != nullptr) recording->push_back({plan.fin_function, plan.fin_grid, plan.block, {buf, buf + n}});
     }
     if (profile) bhhip_event_record(ev1);  // right behind the launches, before the host work below
     ++stats.launches_by_strategy[strategy_name(plan.strategy)];
@@ -1014,7 +1015,7 @@ void EngineHip::runTrial(CachedKernel &ck, const std::vector<bh_base *> &ord2bas
     for (KernelPlan &plan : t.variants[c]) {
         if (plan.function == nullptr) compilePlan(plan);
         for (int o : plan.param_ordinals) ensureResident(ord2base[o]);
-        if (plan.strategy == Strategy::FULL_REDUCE)
+        if (plan.strategy == Strategy::FULL_REDUCE || plan.strategy == Strategy::SEG_REDUCE)
             ensureScratch(reduce_scratch, reduce_scratch_bytes, plan.scratch_bytes, false);
         if (plan.strategy == Strategy::SCAN) ensureScratch(scan_scratch, scan_scratch_bytes, plan.scratch_bytes, true);
     }
