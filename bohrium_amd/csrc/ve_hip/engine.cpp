@@ -647,6 +647,15 @@ std::vector<uint64_t> EngineHip::quietToken() const {
             flush_cache_misses, batch_launches};
 }
 
+// Before a repeat starts: a running repeat holds up to three graphs of the cache (two phases and the
+// multi-period one), so none is destroyed while one runs.
+void EngineHip::trimGraphs() {
+    if (graph_cache.size() + 3 <= 64) return;
+    check(bhhip_synchronize(), "synchronize");
+    for (auto &kv : graph_cache) bhhip_graph_destroy(kv.second);
+    graph_cache.clear();
+}
+
 void *EngineHip::graphFor(const std::vector<IssuedLaunch> &launches) {
     std::string key;
     for (const IssuedLaunch &l : launches) {
@@ -659,11 +668,6 @@ void *EngineHip::graphFor(const std::vector<IssuedLaunch> &launches) {
     }
     auto it = graph_cache.find(key);
     if (it != graph_cache.end()) return it->second;
-    if (graph_cache.size() >= 64) {
-        check(bhhip_synchronize(), "synchronize");
-        for (auto &kv : graph_cache) bhhip_graph_destroy(kv.second);
-        graph_cache.clear();
-    }
     check(bhhip_capture_begin(), "graph capture");
     for (const IssuedLaunch &l : launches) {
         if (bhhip_launch(l.function, l.grid, l.block, l.args.data(), l.args.size()) != 0) {
@@ -1348,6 +1352,7 @@ public:
         const bool with_ext = has_extmethods(*bhir);
         const bool graphable = engine.graph_repeats && !engine.profile && !engine.dry_run && cond == nullptr &&
                                nrepeats >= 4 && !has_slides(*bhir) && !with_ext;
+        if (graphable) engine.trimGraphs();
         struct Iteration {
             std::vector<EngineHip::IssuedLaunch> launches;
             bool quiet;

@@ -130,6 +130,8 @@ public:
     /* Changes whenever the engine allocates device memory, copies between host and device or checks
      * index errors: a repeat iteration whose token is unchanged did nothing but launch kernels. */
     std::vector<uint64_t> quietToken() const;
+    /* Drops the cached graphs when a repeat (up to three graphs) would take them past 64. */
+    void trimGraphs();
     /* A graph holding `launches` in order (captured once per distinct sequence, then cached). */
     void *graphFor(const std::vector<IssuedLaunch> &launches);
     /* Launch a captured graph that stands for `iterations` repeat iterations (for the statistics). */

@@ -157,3 +157,22 @@ def test_repeat_body_replayed_as_period_two_graph(iters):
     assert int(bh.message("graph replays")) > r0, "the repeat body was not replayed as a graph"
     for g, w in zip(got, want):
         assert_parity(g, w, np.float32, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.gpu
+def test_more_repeats_than_cached_graphs():
+    """Thirty grids alive at once, each repeated through its own three graphs (two phases and the multi-period
+    one): the cache of 64 is emptied between repeats, never under a running one."""
+    bh.message("graph: off")
+    want = workloads.jacobi_grid(N)
+    workloads.jacobi_repeat(want, 30)
+    want = want.asnumpy()
+    bh.message("graph: on")
+    grids = [workloads.jacobi_grid(N) for _ in range(30)]
+    before = stat("graph_replays")
+    for G in grids:
+        workloads.jacobi_repeat(G, 30)
+    bh.flush()
+    assert stat("graph_replays") > before and stat("graphs_cached") <= 64
+    for G in grids:
+        np.testing.assert_array_equal(G.asnumpy(), want)
