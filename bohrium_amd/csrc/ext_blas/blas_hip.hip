@@ -10,7 +10,7 @@
  * supplies A[l % 16][l / 16] and B[l / 16][l % 16]; its 4 results are
  * D[4 (l / 16) + r][l % 16] for f32 and D[4 r + l / 16][l % 16] for f64, r = 0..3.
  *
- * Complex types use a 16 x 16 LDS-tiled kernel with complex fused multiply-adds.
+ * Complex types run on the same MFMA tiles, four real products per complex one (gemm_complex).
  */
 #include <hip/hip_runtime.h>
 
@@ -212,8 +212,7 @@ gemm_mfma(const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C, i
             }
 }
 
-// Complex: 16 x 16 threads, each one element of C; K in steps of 16 through LDS.
-template <typename R> struct Cplx {
+template <typename R> struct alignas(2 * sizeof(R)) Cplx {
     R re, im;
 };
 
@@ -233,49 +232,139 @@ template <typename R> __device__ __forceinline__ Cplx<R> msub(Cplx<R> s, Cplx<R>
     return {fma(a.im, x.im, fma(-a.re, x.re, s.re)), fma(-a.im, x.re, fma(-a.re, x.im, s.im))};
 }
 
-// C = alpha op(A) op(B) + beta C with op(B)(k, n) = conj(B[n * ldb + k]) when CONJB; REALDIAG stores
-// the diagonal with a zero imaginary part (Hermitian results).
-template <typename R, bool TA, bool TB, bool CONJB, bool UPPER, bool REALDIAG>
-__global__ void __launch_bounds__(256)
+// Complex on the matrix cores: C = alpha op(A) op(B) + beta C with op(B)(k, n) = conj(B[n * ldb + k]) when
+// CONJB; REALDIAG stores the diagonal with a zero imaginary part (Hermitian results).  Each complex MFMA
+// tile is four real ones (re += ar br, re += (-ai) bi, im += ar bi, im += ai br), so one LDS read of a complex
+// element feeds two operands and the kernel is bound by the MFMA rate: per K step of BK a wave issues
+// TM TN BK MFMAs of 64 (f64) or 32 (f32) cycles for (TM + TN) BK / 4 LDS reads.  Tiles, staging and double
+// buffering as in gemm_mfma; the LDS rows are padded to an odd number of 16-byte elements (c128) or to two
+// 8-byte elements more than a multiple of 16 (c64), so the 16-lane groups of a read fall in disjoint banks.
+// Measured against one FMA thread per element of C: 4096^3 c128 22.8 -> 65.2 TFLOP/s (24.1 -> 8.4 ms), c64
+// 34.6 -> 121 TFLOP/s; 2000 x 1500 x 2500 c128 2678 -> 984 us, 256^3 14.4 -> 14.8 us.
+template <typename R, bool KCONT, int ROWS, int kBK>
+struct CTile {
+    static constexpr int CH = ROWS * kBK / kThreads;
+    static constexpr int KPAD = sizeof(R) == 8 ? 1 : 2;
+    static constexpr int RPAD = sizeof(R) == 8 ? 0 : 16;
+    static constexpr int LDS = KCONT ? ROWS * (kBK + KPAD) : kBK * (ROWS + RPAD);
+    static_assert(CH * kThreads == ROWS * kBK, "tile / thread count");
+
+    static __device__ __forceinline__ void place(int e, int &r, int &k) {
+        const int c = static_cast<int>(threadIdx.x) + e * kThreads;
+        r = KCONT ? c / kBK : c % ROWS;
+        k = KCONT ? c % kBK : c / ROWS;
+    }
+    static __device__ __forceinline__ void fetch(const Cplx<R> *__restrict__ P, int64_t ld, int64_t r0, int64_t k0,
+                                                 int64_t Rn, int64_t K, Cplx<R> *reg) {
+#pragma unroll
+        for (int e = 0; e < CH; ++e) {
+            int r, k;
+            place(e, r, k);
+            const int64_t gr = r0 + r, gk = k0 + k;
+            reg[e] = gr < Rn && gk < K ? P[KCONT ? gr * ld + gk : gk * ld + gr] : Cplx<R>{R(0), R(0)};
+        }
+    }
+    static __device__ __forceinline__ void store(Cplx<R> *lds, const Cplx<R> *reg) {
+#pragma unroll
+        for (int e = 0; e < CH; ++e) {
+            int r, k;
+            place(e, r, k);
+            lds[KCONT ? r * (kBK + KPAD) + k : k * (ROWS + RPAD) + r] = reg[e];
+        }
+    }
+    static __device__ __forceinline__ Cplx<R> read(const Cplx<R> *lds, int r, int k) {
+        return lds[KCONT ? r * (kBK + KPAD) + k : k * (ROWS + RPAD) + r];
+    }
+};
+
+template <typename R, bool TA, bool TB, bool CONJB, bool UPPER, bool REALDIAG, bool SCALED, int TM, int TN, int BK>
+__global__ void __launch_bounds__(kThreads)
 gemm_complex(const Cplx<R> *__restrict__ A, const Cplx<R> *__restrict__ B, Cplx<R> *__restrict__ C, int64_t M,
              int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, R alpha, R beta) {
-    __shared__ Cplx<R> As[16][17];
-    __shared__ Cplx<R> Bs[16][17];
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const int64_t row = static_cast<int64_t>(blockIdx.y) * 16 + ty, col = static_cast<int64_t>(blockIdx.x) * 16 + tx;
-    if (UPPER && static_cast<int64_t>(blockIdx.y) > static_cast<int64_t>(blockIdx.x)) return;  // below the diagonal
-    R sr = 0, si = 0;
-    for (int64_t k0 = 0; k0 < K; k0 += 16) {
-        const int64_t ka = k0 + tx, kb = k0 + ty;
-        Cplx<R> z = {0, 0};
-        As[ty][tx] = (row < M && ka < K) ? (TA ? A[ka * lda + row] : A[row * lda + ka]) : z;
-        if (kb < K && col < N) {
-            const Cplx<R> b = TB ? B[col * ldb + kb] : B[kb * ldb + col];
-            Bs[ty][tx] = CONJB ? conj_of(b) : b;
-        } else {
-            Bs[ty][tx] = z;
-        }
-        __syncthreads();
+    constexpr int BM = 32 * TM, BN = 32 * TN;
+    typedef CTile<R, !TA, BM, BK> ATile;
+    typedef CTile<R, TB, BN, BK> BTile;
+    __shared__ __attribute__((aligned(16))) Cplx<R> As[2][ATile::LDS];
+    __shared__ __attribute__((aligned(16))) Cplx<R> Bs[2][BTile::LDS];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int64_t bm = static_cast<int64_t>(blockIdx.y) * BM, bn = static_cast<int64_t>(blockIdx.x) * BN;
+    if (UPPER && bm > bn + BN - 1) return;  // the whole tile lies below the diagonal
+    const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
+    typename Mfma<R>::Acc re[TM][TN], im[TM][TN];
 #pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const Cplx<R> a = As[ty][k], b = Bs[k][tx];
-            sr = fma(a.re, b.re, sr);
-            sr = fma(-a.im, b.im, sr);
-            si = fma(a.re, b.im, si);
-            si = fma(a.im, b.re, si);
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) re[i][j][r] = im[i][j][r] = R(0);
+    Cplx<R> ra[ATile::CH], rb[BTile::CH];
+    auto fetch = [&](int64_t k0) {
+        ATile::fetch(A, lda, bm, k0, M, K, ra);
+        BTile::fetch(B, ldb, bn, k0, N, K, rb);
+    };
+    fetch(0);
+    ATile::store(As[0], ra);
+    BTile::store(Bs[0], rb);
+    __syncthreads();
+    int buf = 0;
+    for (int64_t k0 = 0; k0 < K; k0 += BK) {
+        const bool more = k0 + BK < K;
+        if (more) fetch(k0 + BK);
+        const Cplx<R> *as = As[buf], *bs = Bs[buf];
+#pragma unroll
+        for (int ks = 0; ks < BK; ks += 4) {
+            const int kr = ks + (lane >> 4);
+            Cplx<R> a[TM], b[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) a[i] = ATile::read(as, wm + i * 16 + (lane & 15), kr);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                b[j] = BTile::read(bs, wn + j * 16 + (lane & 15), kr);
+                if (CONJB) b[j].im = -b[j].im;
+            }
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                const R nai = -a[i].im;
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    re[i][j] = Mfma<R>::step(a[i].re, b[j].re, re[i][j]);
+                    im[i][j] = Mfma<R>::step(a[i].re, b[j].im, im[i][j]);
+                    re[i][j] = Mfma<R>::step(nai, b[j].im, re[i][j]);
+                    im[i][j] = Mfma<R>::step(a[i].im, b[j].re, im[i][j]);
+                }
+            }
         }
+        if (more) {
+            ATile::store(As[buf ^ 1], ra);
+            BTile::store(Bs[buf ^ 1], rb);
+        }
+        // the other buffer is complete, and every wave is done reading this one before it is refilled
         __syncthreads();
+        buf ^= 1;
     }
-    if (row < M && col < N && (!UPPER || row <= col)) {
-        Cplx<R> v = {alpha * sr, alpha * si};
-        if (beta != R(0)) {
-            const Cplx<R> c = C[row * ldc + col];
-            v.re = fma(beta, c.re, v.re);
-            v.im = fma(beta, c.im, v.im);
-        }
-        if (REALDIAG && row == col) v.im = 0;
-        C[row * ldc + col] = v;
-    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int64_t row = bm + wm + i * 16 + Mfma<R>::row(lane, r);
+                const int64_t col = bn + wn + j * 16 + (lane & 15);
+                if (row < M && col < N && (!UPPER || row <= col)) {
+                    Cplx<R> v = {re[i][j][r], im[i][j][r]};
+                    if (SCALED) {
+                        v.re *= alpha;
+                        v.im *= alpha;
+                        if (beta != R(0)) {
+                            const Cplx<R> c = C[row * ldc + col];
+                            v.re = fma(beta, c.re, v.re);
+                            v.im = fma(beta, c.im, v.im);
+                        }
+                    }
+                    if (REALDIAG && row == col) v.im = 0;
+                    C[row * ldc + col] = v;
+                }
+            }
 }
 
 // out (m x m, leading dimension m) from the upper triangle of A (i <= j read, the rest not
@@ -394,12 +483,30 @@ bool launch_real(const Gemm &g) {
     return true;
 }
 
-template <typename R, bool TA, bool TB, bool CONJB, bool UPPER, bool REALDIAG>
-void launch_complex(const Gemm &g) {
-    const dim3 grid(static_cast<unsigned>((g.n + 15) / 16), static_cast<unsigned>((g.m + 15) / 16));
-    gemm_complex<R, TA, TB, CONJB, UPPER, REALDIAG><<<grid, 256, 0, g.s>>>(
+template <typename R, bool TA, bool TB, bool CONJB, bool UPPER, bool REALDIAG, bool SCALED, int TM, int TN, int BK>
+void launch_complex_tiles(const Gemm &g) {
+    const dim3 grid(static_cast<unsigned>((g.n + 32 * TN - 1) / (32 * TN)),
+                    static_cast<unsigned>((g.m + 32 * TM - 1) / (32 * TM)));
+    gemm_complex<R, TA, TB, CONJB, UPPER, REALDIAG, SCALED, TM, TN, BK><<<grid, kThreads, 0, g.s>>>(
         static_cast<const Cplx<R> *>(g.A), static_cast<const Cplx<R> *>(g.B), static_cast<Cplx<R> *>(g.C), g.m, g.n,
         g.k, g.lda, g.ldb, g.ldc, static_cast<R>(g.alpha), static_cast<R>(g.beta));
+}
+
+template <typename R, bool TA, bool TB, bool CONJB, bool UPPER, bool REALDIAG, bool SCALED>
+void launch_complex_scaled(const Gemm &g) {
+    // 64 x 64 tiles when there is a workgroup of them for each of the 256 CUs, else 32 x 32
+    if (((g.m + 63) / 64) * ((g.n + 63) / 64) >= 256)
+        launch_complex_tiles<R, TA, TB, CONJB, UPPER, REALDIAG, SCALED, 2, 2, sizeof(R) == 8 ? 8 : 16>(g);
+    else
+        launch_complex_tiles<R, TA, TB, CONJB, UPPER, REALDIAG, SCALED, 1, 1, 16>(g);
+}
+
+template <typename R, bool TA, bool TB, bool CONJB, bool UPPER, bool REALDIAG>
+void launch_complex(const Gemm &g) {
+    if (g.alpha == 1.0 && g.beta == 0.0)
+        launch_complex_scaled<R, TA, TB, CONJB, UPPER, REALDIAG, false>(g);
+    else
+        launch_complex_scaled<R, TA, TB, CONJB, UPPER, REALDIAG, true>(g);
 }
 
 int launch_status() {

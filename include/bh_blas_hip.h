@@ -24,7 +24,7 @@
  * (bridge/npbackend/bohrium/blas.py:12-117); trmm/trsm write B and ignore C; the
  * front end applies alpha and beta before the call.  Matrices are row-major and
  * C-contiguous; float32 and float64 run on MFMA (v_mfma_f32_16x16x4f32,
- * v_mfma_f64_16x16x4f64), complex64/complex128 on a tiled FMA kernel.
+ * v_mfma_f64_16x16x4f64), complex64/complex128 as four real products on the same.
  *
  * The bhblas_* functions are the same device routines as plain C entry points
  * (device pointers, leading dimensions in elements, the engine stream or any
