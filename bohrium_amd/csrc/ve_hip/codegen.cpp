@@ -343,6 +343,52 @@ struct KernelParam {
     bool is_ptr;
 };
 
+// ---- MAP over tiles: read-only views whose contiguous axis is not the innermost loop's (transposed
+// operands).  In the flat walk each of a wave's lanes reads such a view one row apart: 64 requests of
+// a cache line for 64 elements, bound by the L2 request rate.  Here a workgroup takes a T x T tile of
+// the two axes, copies the transposed views' tile through LDS with its lanes along their contiguous
+// axis, and computes with its lanes along the innermost axis (a row of T + 1 elements in LDS, so
+// neither direction conflicts).  Measured on 4096^2 float32: a.T * 1 64.4 -> 30.7 us (4.4 TB/s),
+// (a + a.T) * 0.5 70.1 -> 39.0 us.
+struct TiledForm {
+    int64_t q = -1;  // the axis along which the transposed views are contiguous
+    std::vector<const bh_view *> views;
+    int side = 0;    // T
+};
+
+// Below this many elements (a few hundred KB, held by the L2s) one round of latency bounds the map either way.
+constexpr uint64_t kTileMinItems = 1u << 16;
+
+TiledForm tiled_form(const std::vector<const LoopB *> &chain, uint64_t p, const std::vector<const bh_view *> &reads) {
+    TiledForm f;
+    if (p < 2) return f;
+    uint64_t total = 1;
+    for (uint64_t r = 0; r < p; ++r) total *= static_cast<uint64_t>(std::max<int64_t>(0, chain[r]->size));
+    if (total < kTileMinItems) return f;
+    const int64_t a = static_cast<int64_t>(p) - 1;
+    int bytes = 0, widest = 1;
+    for (const bh_view *v : reads) {
+        if (v->ndim <= a || v->hasSlide()) continue;
+        if (v->stride[a] == 0 || std::abs(v->stride[a]) < 8) continue;
+        int64_t q = -1;
+        for (int64_t r = 0; r < a; ++r)
+            if (std::abs(v->stride[r]) == 1) q = r;
+        if (q < 0 || (f.q >= 0 && f.q != q)) continue;
+        f.q = q;
+        f.views.push_back(v);
+        const int sz = bh_type_size(v->base->dtype());
+        bytes += sz;
+        widest = std::max(widest, sz);
+    }
+    if (f.views.empty() || chain[a]->size < 32 || chain[f.q]->size < 32) return TiledForm();
+    f.side = 65 * 64 * bytes <= 40960 ? 64 : 32;
+    while (33 * 32 * bytes > 65536) {
+        bytes -= bh_type_size(f.views.back()->base->dtype());
+        f.views.pop_back();
+    }
+    return f;
+}
+
 class Writer {
 public:
     Writer(const LoopB &unit, const WriterConfig &cfg) : unit(unit), cfg(cfg) { collect(); }
@@ -489,6 +535,7 @@ private:
     bool parts = false;
     std::vector<const bh_view *> preloadable(const LoopB &l);
     void emit_map();
+    void emit_map_tiled(const TiledForm &f, const std::vector<const LoopB *> &chain, uint64_t p, const Scope &ksc);
     void emit_row_reduce();
     void emit_seg_reduce();
     void emit_full_reduce();
@@ -1579,6 +1626,92 @@ void Writer::emit_seg_reduce() {
     body << "  }\n";
 }
 
+void Writer::emit_map_tiled(const TiledForm &f, const std::vector<const LoopB *> &chain, uint64_t p, const Scope &ksc) {
+    const int64_t a = static_cast<int64_t>(p) - 1;
+    const int T = f.side, per = T * T / 256, rows = 256 / T;
+    auto n = [&](int64_t r) { return "n" + std::to_string(lid.at(chain[r])); };
+    uint64_t tiles = static_cast<uint64_t>((chain[a]->size + T - 1) / T) * static_cast<uint64_t>((chain[f.q]->size + T - 1) / T);
+    for (int64_t r = 0; r < a; ++r)
+        if (r != f.q) tiles *= static_cast<uint64_t>(chain[r]->size);
+    for (size_t k = 0; k < f.views.size(); ++k)
+        body << "  __shared__ " << hip_type(f.views[k]->base->dtype()) << " tl" << k << "_[" << T * (T + 1) << "];\n";
+    const std::string sT = std::to_string(T), qi = "i" + std::to_string(f.q), ai = "i" + std::to_string(a);
+    body << "  const int64_t ta_ = (" << n(a) << " + " << T - 1 << ") / " << T << ", tb_ = (" << n(f.q) << " + " << T - 1
+         << ") / " << T << ";\n  int64_t tiles_ = ta_ * tb_;\n";
+    for (int64_t r = 0; r < a; ++r)
+        if (r != f.q) body << "  tiles_ *= " << n(r) << ";\n";
+    body << "  const int l_ = threadIdx.x & " << T - 1 << ", w_ = threadIdx.x / " << T << ";\n";
+    body << "  for (int64_t g_ = bh_bid; g_ < tiles_; g_ += bh_nblk) {\n";
+    body << "    int64_t d_ = g_ / ta_;\n    const int64_t a0_ = (g_ - d_ * ta_) * " << T << ";\n";
+    body << "    const int64_t o_ = d_ / tb_;\n    const int64_t b0_ = (d_ - o_ * tb_) * " << T << ";\n    d_ = o_;\n";
+    for (int64_t r = a - 1; r >= 0; --r)
+        if (r != f.q) body << "    const int64_t i" << r << " = d_ % " << n(r) << "; d_ /= " << n(r) << ";\n";
+    std::vector<const bh_view *> others;
+    {
+        std::set<VKey> tiled;
+        for (const bh_view *v : f.views) tiled.insert(vkey(*v));
+        for (const bh_view *v : preloadable(*chain[a]))
+            if (!tiled.count(vkey(*v))) others.push_back(v);
+    }
+    for (int full = 1; full >= 0; --full) {
+        if (full)
+            body << "    if (a0_ + " << T << " <= " << n(a) << " && b0_ + " << T << " <= " << n(f.q) << ") {\n";
+        else
+            body << "    } else {\n";
+        // the tile of every transposed view, lanes along its contiguous axis
+        body << "#pragma unroll\n      for (int k_ = 0; k_ < " << per << "; ++k_) {\n";
+        body << "        const int64_t " << qi << " = b0_ + l_, " << ai << " = a0_ + w_ + k_ * " << rows << ";\n";
+        if (!full) body << "        if (" << qi << " < " << n(f.q) << " && " << ai << " < " << n(a) << ") {\n";
+        for (size_t k = 0; k < f.views.size(); ++k)
+            body << "        tl" << k << "_[(w_ + k_ * " << rows << ") * " << T + 1 << " + l_] = " << ref(ksc, *f.views[k]) << ";\n";
+        if (!full) body << "        }\n";
+        body << "      }\n      __syncthreads();\n";
+        const int U = full ? 4 : 1;
+        body << "      for (int k_ = 0; k_ < " << per << "; k_ += " << U << ") {\n";
+        auto ld = [&](size_t k, int u) { return "ld" + std::to_string(k) + "_" + std::to_string(u); };
+        auto head = [&](int u) {
+            body << "        const int kr_ = w_ + (k_ + " << u << ") * " << rows << ";\n";
+            body << "        const int64_t " << qi << " = b0_ + kr_, " << ai << " = a0_ + l_;\n";
+        };
+        if (full) {
+            for (int u = 0; u < U; ++u)
+                for (size_t k = 0; k < others.size(); ++k)
+                    body << "        " << hip_type(others[k]->base->dtype()) << " " << ld(k, u) << ";\n";
+            for (int u = 0; u < U && !others.empty(); ++u) {
+                body << "        {\n";
+                head(u);
+                for (size_t k = 0; k < others.size(); ++k) body << "        " << ld(k, u) << " = " << ref(ksc, *others[k]) << ";\n";
+                body << "        }\n";
+            }
+        }
+        for (int u = 0; u < U; ++u) {
+            Scope pre;
+            pre.parent = &ksc;
+            for (size_t k = 0; k < f.views.size(); ++k)
+                pre.preload[vkey(*f.views[k])] = "tl" + std::to_string(k) + "_[l_ * " + std::to_string(T + 1) + " + kr_]";
+            if (full)
+                for (size_t k = 0; k < others.size(); ++k) pre.preload[vkey(*others[k])] = ld(k, u);
+            body << "        {\n";
+            head(u);
+            if (!full) body << "        if (" << qi << " < " << n(f.q) << " && " << ai << " < " << n(a) << ") {\n";
+            std::vector<Scope> scopes(p);
+            const Scope *parent = &pre;
+            for (uint64_t r = 0; r < p; ++r) {
+                scopes[r].parent = parent;
+                declare_scope(*chain[r], scopes[r], 5);
+                if (r == p - 1) emit_blocks(*chain[r], scopes[r], 5);
+                parent = &scopes[r];
+            }
+            for (int64_t r = a; r >= 0; --r) write_back(*chain[r], scopes[r], 5);
+            if (!full) body << "        }\n";
+            body << "        }\n";
+        }
+        body << "      }\n";
+    }
+    body << "    }\n    __syncthreads();\n  }\n";
+    kp.grid = std::max<uint64_t>(1, std::min<uint64_t>(tiles, 4 * static_cast<uint64_t>(cfg.max_grid)));
+}
+
 // ---- MAP: grid-stride over the flattened leading parallel ranks
 void Writer::emit_map() {
     const LoopB &l0 = unit._block_list.back().getLoop();
@@ -1595,6 +1728,15 @@ void Writer::emit_map() {
     body << ";\n";
     // Only loops without inner sequential work are unrolled (their body is straight-line code).
     const bool flat = p == 1 ? l0.isInnermost() : chain[p - 1]->isInnermost();
+    if (flat && p > 1) {
+        const TiledForm f = tiled_form(chain, p, preloadable(*chain[p - 1]));
+        if (!f.views.empty()) {
+            // (tot_ is not used: the tiles are counted instead)
+            emit_map_tiled(f, chain, p, ksc);
+            write_back(unit, ksc, 1);
+            return;
+        }
+    }
     Element e;
     e.outer = &ksc;
     e.body_loop = flat ? chain[p - 1] : nullptr;
