@@ -361,7 +361,9 @@ void EngineHip::exchangeTwin(const TwinUpdate &u) {
     std::swap(g.ptr, t.ptr);
     noteWrite(u.target, g);
     noteWrite(u.twin, t);
-    twins[u.target].in_step_at = u.in_step_after ? g.writes : ~0ull;
+    Twin &tw = twins[u.target];
+    tw.in_step_at = u.in_step_after ? g.writes : ~0ull;
+    tw.region = u.region;
     flush_exchanges.push_back(u);
     ++twin_exchanges;
 }
@@ -732,10 +734,12 @@ void EngineHip::handleExecution(BhIR *bhir) {
             if (!tw.base) tw.base.reset(new bh_base(g->nelem(), g->dtype()));
             return tw.base.get();
         };
-        auto in_step = [&](bh_base *g) {
+        auto in_step = [&](const bh_view &c) {
+            const bh_base *g = c.base;
             auto tw = twins.find(g);
             auto b = bufs.find(g);
-            return tw != twins.end() && b != bufs.end() && tw->second.in_step_at == b->second.writes;
+            return tw != twins.end() && b != bufs.end() && tw->second.in_step_at == b->second.writes &&
+                   tw->second.region == c;
         };
         exchanges = rewrite_in_place_updates(instr_list, rewrite_store, syncs, twin_for, in_step);
         for (const TwinUpdate &u : exchanges) twin_full_copies += u.full_copy ? 1 : 0;

@@ -202,11 +202,12 @@ private:
     bool resident = true;
     int num_cus = 0;  // compute units of the device (0 in compile-only mode)
     std::unordered_map<const bh_base *, DeviceBuffer> bufs;
-    /* The second buffer of an array updated in place (rewrite_in_place_updates), and the write
-     * count of the array at which the twin last equalled it outside the updated view. */
+    /* The second buffer of an array updated in place (rewrite_in_place_updates), the write count of
+     * the array at which the twin last equalled it outside the updated view, and that view. */
     struct Twin {
         std::unique_ptr<bh_base> base;
         uint64_t in_step_at = ~0ull;
+        bh_view region;
     };
     std::unordered_map<const bh_base *, Twin> twins;
     std::set<bh_base *> flush_written;

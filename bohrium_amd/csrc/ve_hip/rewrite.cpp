@@ -128,7 +128,7 @@ constexpr size_t kNone = static_cast<size_t>(-1);
 std::vector<TwinUpdate> rewrite_in_place_updates(std::vector<bh_instruction *> &list, RewriteStore &store,
                                                  const std::set<bh_base *> &syncs,
                                                  const std::function<bh_base *(bh_base *)> &twin_for,
-                                                 const std::function<bool(bh_base *)> &in_step) {
+                                                 const std::function<bool(const bh_view &)> &in_step) {
     std::vector<TwinUpdate> out;
     for (const bh_instruction *i : list) {
         if (i->opcode > BH_MAX_OPCODE_ID) return out;
@@ -177,9 +177,10 @@ std::vector<TwinUpdate> rewrite_in_place_updates(std::vector<bh_instruction *> &
             u.target = G;
             u.twin = twin;
             u.temp = T;
+            u.region = V;
             bool written_before = false;
             for (size_t k = 0; k < p0; ++k) written_before |= writes(list[k], G);
-            u.full_copy = written_before || !in_step(G);
+            u.full_copy = written_before || !in_step(V);
             u.in_step_after = true;
             for (size_t k = q + 1; k < list.size(); ++k) u.in_step_after &= !writes(list[k], G);
 

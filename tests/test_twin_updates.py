@@ -176,3 +176,47 @@ def test_more_repeats_than_cached_graphs():
     assert stat("graph_replays") > before and stat("graphs_cached") <= 64
     for G in grids:
         np.testing.assert_array_equal(G.asnumpy(), want)
+
+
+OTHER_REGION = r"""
+import sys
+sys.path.insert(0, %(root)r)
+import bohrium_amd as bh
+G = bh.zeros((1024, 1024))
+bh.flush()
+def update(lo):
+    c = G[lo:-lo, lo:-lo]
+    c[...] = (G[lo - 1:-lo - 1, lo:-lo] + c) * 0.5
+    bh.flush()
+for lo in (1, 1, 2, 2, 1):
+    update(lo)
+    print([l.split()[1] for l in bh.message("statistic").splitlines() if l.startswith("twin_full_copies")][0])
+"""
+
+
+def test_a_twin_is_in_step_for_its_own_view_only():
+    """After an update of c the twin equals G outside c; an update of another view copies G first."""
+    r = subprocess.run([sys.executable, "-c", OTHER_REGION % {"root": ROOT}], env=dict(os.environ, BH_HIP_DRY_RUN="1"),
+                       stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout[-3000:]
+    assert [int(l) for l in r.stdout.split()] == [1, 1, 2, 2, 3], r.stdout
+
+
+@pytest.mark.gpu
+def test_updates_of_different_views():
+    """A whole-array update (the last copy of a converted array is one) and updates of two interiors."""
+    def program():
+        G = (bh.random.RandomState(3).random123((N * N,)) % np.uint64(100)).astype(np.float64).astype(np.float64)
+        G = G.reshape((N, N))
+        bh.flush()
+        out = []
+        for lo in (1, 2, 1, 3, 3):
+            c = G[lo:-lo, lo:-lo]
+            c[...] = (G[lo - 1:-lo - 1, lo:-lo] + G[lo:-lo, lo - 1:-lo - 1] + c) * 0.5
+            bh.flush()
+            out.append(G.copy())
+            bh.flush()
+        return out
+    got, want = run_both(program)
+    for g, w in zip(got, want):
+        np.testing.assert_array_equal(g, w)
