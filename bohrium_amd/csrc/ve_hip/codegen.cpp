@@ -533,6 +533,10 @@ private:
      * stencil's neighbouring rows are read by the workgroups of one L2. */
     void grid_stride(const std::string &tot, int unroll, const Element &e);
     bool parts = false;
+    /* A 2-D stencil's walk by column groups and row bands; false (nothing emitted) when the body is none.
+     * Sets the number of thread tasks. */
+    bool stencil_walk(const Element &e, const std::string &n0, const std::string &n1, int64_t s0, int64_t s1, int unroll,
+                      int64_t *tasks);
     std::vector<const bh_view *> preloadable(const LoopB &l);
     void emit_map();
     void emit_map_tiled(const TiledForm &f, const std::vector<const LoopB *> &chain, uint64_t p, const Scope &ksc);
@@ -895,6 +899,197 @@ bool shifted_reads(const LoopB &l) {
     return false;
 }
 } // namespace
+
+// ---- stencil walk of a 2-D iteration (i0 of s0, i1 of s1): neighbouring elements of one array read through
+// several views.  Element by element each view is a load of its own (5 loads of 4 bytes and their index
+// arithmetic per point of a 5-point stencil: about 60 VALU instructions, which bounded the sweep at half the
+// copy rate).  Here a thread owns V neighbouring columns and walks down a band of rows with a window of the
+// array in registers: every element of the band is loaded once per thread (16-byte loads of the V columns
+// plus the side columns), and a group of `ur` rows is loaded before it is computed.  Measured on the 8192^2
+// float32 5-point sweep with max|new - old|: 133 -> 106 us (4.0 -> 5.1 TB/s; a plain copy reaches 5.6), 200 sweeps
+// 27.3 -> 21.9 ms.
+namespace {
+// A window: the views of one base with equal strides, as offsets (row, column) from the first.
+struct Window {
+    const bh_view *first = nullptr;
+    std::map<VKey, std::pair<int, int> > taps;
+    std::vector<const bh_view *> views;
+};
+
+// Windows of the read-only views `reads` of a 2-D loop nest (two or more views each, unit column stride,
+// offsets within 3 rows and 8 columns).
+std::vector<Window> stencil_windows(const std::vector<const bh_view *> &reads) {
+    std::vector<Window> out;
+    for (const bh_view *v : reads) {
+        if (v->ndim != 2 || v->stride[1] != 1 || v->hasSlide() || v->stride[0] < 16) continue;
+        bool placed = false;
+        for (Window &w : out) {
+            if (w.first->base != v->base || w.first->stride[0] != v->stride[0]) continue;
+            const int64_t s0 = v->stride[0], d = v->start - w.first->start;
+            const int64_t dr = d >= 0 ? (d + s0 / 2) / s0 : -((-d + s0 / 2) / s0), dc = d - dr * s0;
+            if (std::abs(dr) > 3 || std::abs(dc) > 8) continue;
+            w.taps[vkey(*v)] = {static_cast<int>(dr), static_cast<int>(dc)};
+            w.views.push_back(v);
+            placed = true;
+            break;
+        }
+        if (placed) continue;
+        Window w;
+        w.first = v;
+        w.taps[vkey(*v)] = {0, 0};
+        w.views.push_back(v);
+        out.push_back(w);
+    }
+    out.erase(std::remove_if(out.begin(), out.end(), [](const Window &w) { return w.taps.size() < 2; }), out.end());
+    return out;
+}
+
+// Fewer elements than this (2^20: 1024^2, 256 workgroups of single row groups) leave too few bands to fill the chip,
+// and their arrays stay in the L2s, where the element walk's repeated loads are cheap.
+constexpr int64_t kStencilMinItems = 1 << 20;
+} // namespace
+
+bool Writer::stencil_walk(const Element &e, const std::string &n0, const std::string &n1, int64_t s0, int64_t s1,
+                          int unroll, int64_t *tasks) {
+    if (e.body_loop == nullptr || s0 * s1 < kStencilMinItems || s0 * s1 >= (1ll << 31) || s1 < 64) return false;
+    const std::vector<const bh_view *> reads = preloadable(*e.body_loop);
+    const std::vector<Window> wins = stencil_windows(reads);
+    if (wins.empty()) return false;
+    std::vector<const bh_view *> others;
+    int widest = 1;
+    for (const bh_view *v : reads) {
+        widest = std::max(widest, bh_type_size(v->base->dtype()));
+        bool in = false;
+        for (const Window &w : wins) in |= w.taps.count(vkey(*v)) != 0;
+        if (!in) others.push_back(v);
+    }
+    const int V = std::max(1, std::min(4, 16 / widest));
+    const int UR = std::max(2, std::min(8, unroll));
+    if (s1 / V < 16) return false;
+    // Bands of up to 8 row groups, fewer when the bands would not give every CU 8 workgroups.
+    const int64_t groups = s1 / V;
+    int64_t H = 8 * UR;
+    while (H > UR && ((s0 + H - 1) / H) * groups < 256ll * 8 * kp.block) H -= UR;
+    shape_args.emplace_back("st_h", H);
+    *tasks = (s0 + H - 1) / H * groups;
+
+    // Columns of window k that row j of a row group needs: those of the taps that touch it.
+    auto need = [&](const Window &w, int j) {
+        std::set<int> c;
+        for (const auto &t : w.taps)
+            if (j - t.second.first >= 0 && j - t.second.first < UR)
+                for (int v = 0; v < V; ++v) c.insert(t.second.second + v);
+        return c;
+    };
+    auto reg = [](size_t k, int j, int c) {
+        auto num = [](int x) { return (x < 0 ? "m" : "p") + std::to_string(std::abs(x)); };
+        return "w" + std::to_string(k) + "_" + num(j) + "_" + num(c);
+    };
+    auto load = [&](int ind, size_t k, int j, int c, const std::string &row) {
+        const bh_view &v = *wins[k].first;
+        indent(body, ind);
+        body << reg(k, j, c) << " = a" << bid.at(v.base) << "[vo" << os_id(v) << " + (" << row << " + " << j << ") * vs"
+             << stride_id(v.stride[0]) << " + (c0_ + " << c << ")];\n";
+    };
+    body << "  const int64_t ng_ = " << n1 << " / " << V << ", nt_ = (" << n0 << " + st_h - 1) / st_h * ng_;\n";
+    if (parts) {
+        body << "  const unsigned px_ = bh_nblk < BH_XCDS ? bh_nblk : BH_XCDS;\n";
+        body << "  const unsigned pw_ = bh_nblk / px_ + (bh_bid % px_ < bh_nblk % px_ ? 1u : 0u);\n";
+        body << "  const int64_t pt_ = ((nt_ + px_ - 1) / px_ + BH_WG - 1) / BH_WG * BH_WG;\n";
+        body << "  const int64_t p0_ = (int64_t)(bh_bid % px_) * pt_;\n";
+        body << "  const int64_t pe_ = p0_ + pt_ < nt_ ? p0_ + pt_ : nt_;\n";
+        body << "  const int64_t st_ = (int64_t)pw_ * BH_WG;\n";
+        body << "  int64_t g_ = p0_ + (int64_t)(bh_bid / px_) * BH_WG + threadIdx.x;\n";
+    } else {
+        body << "  const int64_t pe_ = nt_, st_ = (int64_t)bh_nblk * BH_WG;\n";
+        body << "  int64_t g_ = (int64_t)bh_bid * BH_WG + threadIdx.x;\n";
+    }
+    body << "  for (; g_ < pe_; g_ += st_) {\n";
+    body << "    const int64_t b_ = (int64_t)((uint32_t)g_ / (uint32_t)ng_), c0_ = (g_ - b_ * ng_) * " << V << ";\n";
+    body << "    int64_t r_ = b_ * st_h;\n    const int64_t re_ = r_ + st_h < " << n0 << " ? r_ + st_h : " << n0 << ";\n";
+    body << "    if (r_ + " << UR << " <= re_) {\n";
+    struct Span {
+        int lo, hi;
+    };
+    std::vector<Span> span;
+    for (size_t k = 0; k < wins.size(); ++k) {
+        Span s{0, 0};
+        for (const auto &t : wins[k].taps) {
+            s.lo = std::min(s.lo, t.second.first);
+            s.hi = std::max(s.hi, t.second.first);
+        }
+        span.push_back(s);
+        const std::string T = hip_type(wins[k].first->base->dtype());
+        // the rows that a group takes over from the one before it
+        for (int j = s.lo; j < s.hi; ++j)
+            for (int c : need(wins[k], j)) body << "      " << T << " " << reg(k, j, c) << ";\n";
+        for (int j = s.lo; j < s.hi; ++j) {
+            const std::set<int> have = need(wins[k], j + UR);
+            for (int c : need(wins[k], j))
+                if (have.count(c)) load(3, k, j, c, "r_");
+        }
+    }
+    body << "      for (; r_ + " << UR << " <= re_; r_ += " << UR << ") {\n";
+    for (size_t k = 0; k < wins.size(); ++k) {
+        const std::string T = hip_type(wins[k].first->base->dtype());
+        for (int j = span[k].hi; j < UR + span[k].hi; ++j)
+            for (int c : need(wins[k], j)) body << "        " << T << " " << reg(k, j, c) << ";\n";
+        for (int j = span[k].lo; j < UR + span[k].hi; ++j) {
+            const std::set<int> have = j < span[k].hi ? need(wins[k], j + UR) : std::set<int>();
+            for (int c : need(wins[k], j))
+                if (!have.count(c)) load(4, k, j, c, "r_");
+        }
+    }
+    auto ld = [&](size_t k, int u, int v) {
+        return "ld" + std::to_string(k) + "_" + std::to_string(u) + "_" + std::to_string(v);
+    };
+    auto at = [&](int u, int v) {
+        body << "        {\n          const int64_t i0 = r_ + " << u << ", i1 = c0_ + " << v << ";\n";
+    };
+    for (size_t k = 0; k < others.size(); ++k)
+        for (int u = 0; u < UR; ++u)
+            for (int v = 0; v < V; ++v)
+                body << "        " << hip_type(others[k]->base->dtype()) << " " << ld(k, u, v) << ";\n";
+    for (int u = 0; u < UR; ++u)
+        for (int v = 0; v < V && !others.empty(); ++v) {
+            at(u, v);
+            for (size_t k = 0; k < others.size(); ++k) body << "          " << ld(k, u, v) << " = " << ref(*e.outer, *others[k]) << ";\n";
+            body << "        }\n";
+        }
+    for (int u = 0; u < UR; ++u)
+        for (int v = 0; v < V; ++v) {
+            Scope pre;
+            pre.parent = e.outer;
+            for (size_t k = 0; k < others.size(); ++k) pre.preload[vkey(*others[k])] = ld(k, u, v);
+            for (size_t k = 0; k < wins.size(); ++k)
+                for (const auto &t : wins[k].taps)
+                    pre.preload[t.first] = reg(k, u + t.second.first, v + t.second.second);
+            at(u, v);
+            e.compute(5, &pre);
+            body << "        }\n";
+        }
+    for (size_t k = 0; k < wins.size(); ++k)
+        for (int j = span[k].lo; j < span[k].hi; ++j) {
+            const std::set<int> have = need(wins[k], j + UR);
+            for (int c : need(wins[k], j))
+                if (have.count(c)) body << "        " << reg(k, j, c) << " = " << reg(k, j + UR, c) << ";\n";
+        }
+    body << "      }\n    }\n";
+    // the band's last rows, element by element
+    body << "    for (; r_ < re_; ++r_)\n      for (int v_ = 0; v_ < " << V << "; ++v_) {\n        const int64_t i0 = r_, i1 = c0_ + v_;\n";
+    e.compute(4, e.outer);
+    body << "      }\n  }\n";
+    if (V > 1) {
+        // the columns past the last whole group
+        body << "  const int64_t cr_ = " << n1 << " - ng_ * " << V << ";\n";
+        body << "  if (cr_ > 0)\n    for (int64_t f_ = (int64_t)bh_bid * BH_WG + threadIdx.x; f_ < cr_ * " << n0
+             << "; f_ += (int64_t)bh_nblk * BH_WG) {\n";
+        body << "      const int64_t i0 = f_ / cr_, i1 = ng_ * " << V << " + (f_ - i0 * cr_);\n";
+        e.compute(3, e.outer);
+        body << "    }\n";
+    }
+    return true;
+}
 
 void Writer::grid_stride(const std::string &tot_in, int unroll, const Element &e) {
     std::string tot = tot_in;
@@ -1777,6 +1972,15 @@ void Writer::emit_map() {
         }
     };
     parts = cfg.xcd_parts && shifted_reads(l0);
+    int64_t tasks = 0;
+    if (p == 2 && parts &&
+        stencil_walk(e, "n" + std::to_string(lid.at(chain[0])), "n" + std::to_string(lid.at(chain[1])), chain[0]->size,
+                     chain[1]->size, cfg.map_unroll, &tasks)) {
+        parts = false;
+        write_back(unit, ksc, 1);
+        kp.grid = std::max<uint64_t>(1, std::min<uint64_t>((static_cast<uint64_t>(tasks) + kp.block - 1) / kp.block, cfg.max_grid));
+        return;
+    }
     grid_stride("tot_", flat ? cfg.map_unroll : 1, e);
     parts = false;
     write_back(unit, ksc, 1);
@@ -1953,7 +2157,9 @@ void Writer::emit_full_reduce() {
             write_back(*l1, sc, ind);
         };
         parts = cfg.xcd_parts && shifted_reads(l0);
-        grid_stride("tot_", cfg.reduce_unroll, e);
+        int64_t tasks = 0;
+        if (!(parts && stencil_walk(e, n0, n1, l0.size, l1->size, cfg.reduce_unroll, &tasks)))
+            grid_stride("tot_", cfg.reduce_unroll, e);
         parts = false;
     } else {
         Element e;
