@@ -2253,6 +2253,25 @@ void Writer::emit_scan() {
     const std::string T = hip_type(t);
     const int items = cfg.scan_items;
     const int64_t tile_elems = static_cast<int64_t>(kp.block) * items;
+    // V neighbours per thread when every array is walked contiguously (16 bytes of the widest input)
+    int V = 1;
+    {
+        bool unit = true;
+        int widest = 1;
+        for (const InstrPtr &i : jitk::allInstr(l0)) {
+            if (bh_opcode_is_system(i->opcode)) continue;
+            for (size_t o = 0; o < i->operand.size(); ++o) {
+                const bh_view &v = i->operand[o];
+                if (v.isConstant() || (i->opcode == BH_GATHER && o == 1) || v.ndim < 1) continue;
+                unit &= v.ndim == 1 && (v.stride[0] == 1 || v.stride[0] == 0 || v.shape[0] == 1);
+                if (o > 0 && std::find(kp.params.begin(), kp.params.end(), v.base) != kp.params.end())
+                    widest = std::max(widest, bh_type_size(v.base->dtype()));
+            }
+        }
+        if (unit) V = std::max(1, std::min(4, 16 / widest));
+        while (items % V != 0) V /= 2;
+    }
+    const int groups = items / V;
     const int64_t ntiles = (l0.size + tile_elems - 1) / tile_elems;
     kp.grid = static_cast<uint64_t>(std::max<int64_t>(1, ntiles));
     // Scratch layout: [tile counter u64 = epoch << 32 | tiles taken, pad to 256], then one record
@@ -2287,15 +2306,19 @@ void Writer::emit_scan() {
     body << "  " << T << " v_[" << items << "];\n";
     Scope ksc;
     declare_scope(unit, ksc, 1);
-    // The elements first (every load of the tile issued before the first wave scan waits for one):
-    // a full tile without bounds checks, unrolled; the last tile with them.
+    // A thread owns `groups` runs of V neighbouring elements: 16-byte loads where the views are
+    // contiguous, and one wave scan per run instead of one per element.  The elements first (every load of
+    // the tile issued before the first wave scan waits for one): a full tile without bounds checks, the
+    // last tile with them; both unrolled, so that v_ stays in registers.  Measured: the int64 running count of
+    // 6e7 float32 276 -> 195 us (one element per thread and wave scan, 16 per tile and thread, before; 64 now).
     for (int full = 1; full >= 0; --full) {
         if (full)
-            body << "  if (tb_ + " << tile_elems << " <= n" << lid.at(&l0) << ") {\n#pragma unroll\n";
+            body << "  if (tb_ + " << tile_elems << " <= n" << lid.at(&l0) << ") {\n";
         else
             body << "  } else {\n";
-        body << "  for (int j_ = 0; j_ < " << items << "; ++j_) {\n";
-        body << "    const int64_t i0 = tb_ + ((int64_t)wave_ * " << items << " + j_) * 64 + lane_;\n";
+        body << "#pragma unroll\n  for (int j_ = 0; j_ < " << groups << "; ++j_) {\n";
+        body << "#pragma unroll\n  for (int e_ = 0; e_ < " << V << "; ++e_) {\n";
+        body << "    const int64_t i0 = tb_ + (((int64_t)wave_ * " << groups << " + j_) * 64 + lane_) * " << V << " + e_;\n";
         body << "    " << T << " x_ = " << ident << ";\n";
         body << (full ? "    {\n" : "    if (i0 < n" + std::to_string(lid.at(&l0)) + ") {\n");
         {
@@ -2305,14 +2328,18 @@ void Writer::emit_scan() {
             emit_blocks(l0, sc, 3);
             write_back(l0, sc, 3);
         }
-        body << "    }\n    v_[j_] = x_;\n  }\n";
+        body << "    }\n    v_[j_ * " << V << " + e_] = x_;\n  }\n  }\n";
     }
     body << "  }\n";
-    body << "  " << T << " carry_ = " << ident << ";\n";
-    body << "  for (int j_ = 0; j_ < " << items << "; ++j_) {\n";
-    body << "    const " << T << " x_ = op_(carry_, bh_wave_inclusive_scan(v_[j_], op_));\n";
-    body << "    carry_ = bh_lane(x_, 63);\n";
-    body << "    v_[j_] = x_;\n  }\n";
+    // Prefixes inside a run by the thread, of the runs across the wave, and carried from row to row.
+    body << "  " << T << " carry_ = " << ident << ", g_[" << groups << "];\n";
+    body << "#pragma unroll\n  for (int j_ = 0; j_ < " << groups << "; ++j_) {\n";
+    body << "#pragma unroll\n    for (int e_ = 1; e_ < " << V << "; ++e_) v_[j_ * " << V << " + e_] = op_(v_[j_ * " << V
+         << " + e_ - 1], v_[j_ * " << V << " + e_]);\n";
+    body << "    " << T << " tot_;\n";
+    body << "    const " << T << " ex_ = bh_wave_exclusive_scan(v_[j_ * " << V << " + " << V - 1 << "], op_, " << T << "(" << ident
+         << "), &tot_);\n";
+    body << "    g_[j_] = op_(carry_, ex_);\n    carry_ = op_(carry_, tot_);\n  }\n";
     body << "  if (lane_ == 63) bh_wtot_[wave_] = carry_;\n  __syncthreads();\n";
     body << "  " << T << " wpre_ = " << ident << ", ttot_ = " << ident << ";\n";
     body << "  for (int w_ = 0; w_ < BH_WAVES; ++w_) { if (w_ < wave_) wpre_ = op_(wpre_, bh_wtot_[w_]); ttot_ = op_(ttot_, bh_wtot_[w_]); }\n";
@@ -2349,9 +2376,14 @@ void Writer::emit_scan() {
     body << "  __syncthreads();\n";
     body << "  const " << T << " pre_ = op_(bh_excl_s, wpre_);\n";
     const bh_view &out = acc->operand[0];
-    body << "  for (int j_ = 0; j_ < " << items << "; ++j_) {\n";
-    body << "    const int64_t i0 = tb_ + ((int64_t)wave_ * " << items << " + j_) * 64 + lane_;\n";
-    body << "    if (i0 < n" << lid.at(&l0) << ") a" << bid.at(out.base) << "[" << index(out) << "] = op_(pre_, v_[j_]);\n";
+    for (int full = 1; full >= 0; --full) {
+        body << (full ? "  if (tb_ + " + std::to_string(tile_elems) + " <= n" + std::to_string(lid.at(&l0)) + ") {\n" : "  } else {\n");
+        body << "#pragma unroll\n  for (int j_ = 0; j_ < " << groups << "; ++j_) {\n    const " << T << " p_ = op_(pre_, g_[j_]);\n";
+        body << "#pragma unroll\n  for (int e_ = 0; e_ < " << V << "; ++e_) {\n";
+        body << "    const int64_t i0 = tb_ + (((int64_t)wave_ * " << groups << " + j_) * 64 + lane_) * " << V << " + e_;\n";
+        body << (full ? "    " : "    if (i0 < n" + std::to_string(lid.at(&l0)) + ") ") << "a" << bid.at(out.base) << "["
+             << index(out) << "] = op_(p_, v_[j_ * " << V << " + e_]);\n  }\n  }\n";
+    }
     body << "  }\n";
     write_back(unit, ksc, 1);
 }

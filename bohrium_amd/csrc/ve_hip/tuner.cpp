@@ -89,7 +89,7 @@ std::vector<LaunchKnobs> Tuner::candidates(Strategy s, const LaunchKnobs &base) 
             }
             break;
         case Strategy::SCAN:
-            for (int items : {4, 8, 16}) {
+            for (int items : {4, 8, 16, 32, 64}) {
                 LaunchKnobs k = base;
                 k.scan_items = items;
                 add(k);
