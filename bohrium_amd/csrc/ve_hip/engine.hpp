@@ -391,6 +391,15 @@ private:
     void ensureScratch(unsigned char *&ptr, uint64_t &have, uint64_t need, bool zero);
 
     void checkErrors();
+    /* Raises the errors of a non-zero flag value and clears the device's flag. */
+    void raiseErrors(unsigned int flag);
+    /* Small device arrays to the host in one launch and one wait: a kernel writes every base of `bases`
+     * that is newer on the device and holds at most kFetchBytes, and the error flag when it is due
+     * (`flag`, or raised without a check since), into page-locked staging.  Other bases are left alone. */
+    void fetchSmall(const std::vector<bh_base *> &bases, bool flag);
+    static constexpr uint64_t kFetchBytes = 64 << 10, kFetchArena = 2 << 20;
+    unsigned char *fetch_staging = nullptr;  // kFetchArena bytes, page-locked, for the engine's lifetime
+    void *fetch_fn = nullptr;
 };
 
 } // namespace vehip
