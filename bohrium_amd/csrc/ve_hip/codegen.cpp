@@ -1473,6 +1473,7 @@ SegForm seg_form(const LoopB &l0, const std::set<const bh_base *> &params) {
         for (size_t o = 1; o < i->operand.size(); ++o) {
             const bh_view &v = i->operand[o];
             if (v.isConstant() || !params.count(v.base) || v.ndim <= c || !seen.insert(vkey(v)).second) continue;
+            if (v.stride[c] == 0 || v.stride[a] == 0) continue;  // (broadcast: a fraction of the elements)
             const int sz = bh_type_size(v.base->dtype());
             if (v.stride[c] == 1 && v.shape[c] > 1 && v.stride[a] != 1) {
                 rows += sz;
@@ -2646,6 +2647,54 @@ std::vector<LoopB> fold_serial_tails(std::vector<LoopB> kernels) {
 }
 
 namespace {
+// The bases a unit addresses as arrays (its writer's parameters).
+std::set<const bh_base *> param_bases(const LoopB &unit) {
+    std::set<const bh_base *> out;
+    for (const bh_base *b : unit.getAllNonTemps()) out.insert(b);
+    return out;
+}
+
+// The position of a kernel's only computing block when that is a loop, else -1.
+int only_loop(const LoopB &kernel) {
+    int at = -1;
+    for (size_t k = 0; k < kernel._block_list.size(); ++k) {
+        const Block &b = kernel._block_list[k];
+        if (b.isSystemOnly()) continue;
+        if (b.isInstr() || at >= 0) return -1;
+        at = static_cast<int>(k);
+    }
+    return at;
+}
+} // namespace
+
+std::vector<LoopB> fold_row_tails(std::vector<LoopB> kernels) {
+    std::vector<LoopB> out;
+    for (LoopB &k : kernels) {
+        const int b = only_loop(k);
+        const int a = out.empty() ? -1 : only_loop(out.back());
+        bool folded = false;
+        if (a >= 0 && b >= 0) {
+            const LoopB &la = out.back()._block_list[a].getLoop(), &lb = k._block_list[b].getLoop();
+            if (la.rank == 0 && lb.rank == 0 && la.size == lb.size && lb.isInnermost() && lb._sweeps.empty() &&
+                seg_form(la, param_bases(out.back())).C != nullptr &&
+                jitk::mergeable(out.back()._block_list[a], k._block_list[b], false)) {
+                LoopB merged = out.back();
+                merged._block_list[a] = Block(jitk::merge(la, lb));
+                for (size_t i = 0; i < k._block_list.size(); ++i)
+                    if (static_cast<int>(i) != b) merged._block_list.push_back(k._block_list[i]);
+                merged.metadataUpdate();
+                if (seg_form(merged._block_list[a].getLoop(), param_bases(merged)).C != nullptr) {
+                    out.back() = std::move(merged);
+                    folded = true;
+                }
+            }
+        }
+        if (!folded) out.push_back(std::move(k));
+    }
+    return out;
+}
+
+namespace {
 // Every operand dimension of every instruction must be iterated by the enclosing loop of the
 // matching rank, and that loop may not run past the dimension (the generated index is
 // start + sum(i_rank * stride), in bounds only then).  `sizes` holds the enclosing loop sizes
@@ -2696,15 +2745,6 @@ std::string verify_kernel(const LoopB &kernel) {
     verify_loop_ranks(kernel, sizes, err);
     return err;
 }
-
-namespace {
-// The bases a unit addresses as arrays (its writer's parameters).
-std::set<const bh_base *> param_bases(const LoopB &unit) {
-    std::set<const bh_base *> out;
-    for (const bh_base *b : unit.getAllNonTemps()) out.insert(b);
-    return out;
-}
-} // namespace
 
 std::vector<KernelPlan> plan_kernel(const LoopB &kernel, const WriterConfig &cfg) {
     std::vector<KernelPlan> ret;

@@ -122,6 +122,11 @@ struct WriterConfig {
  * that one ends in a FULL_REDUCE loop: its finalize kernel then runs them. */
 std::vector<jitk::LoopB> fold_serial_tails(std::vector<jitk::LoopB> kernels);
 
+/* Append each map over the outputs of the segmented reduction before it (the division of a column mean) to that
+ * reduction's loop: it then runs with the finalized outputs, in their registers.  (The fuser has no chance
+ * to: the loops have one shape only after the reduction was pushed inwards.) */
+std::vector<jitk::LoopB> fold_row_tails(std::vector<jitk::LoopB> kernels);
+
 /* Check that every operand dimension is iterated within its extent by the loop of the matching
  * rank (what the generated indexing assumes); returns "" or a description of each violation. */
 std::string verify_kernel(const jitk::LoopB &kernel);

@@ -171,6 +171,7 @@ EngineHip::EngineHip(component::ComponentVE &comp) : comp(comp) {
     wcfg.xcd_remap = cfg.defaultGet<bool>("xcd_remap", false);
     wcfg.xcd_parts = cfg.defaultGet<bool>("xcd_parts", true);
     unflatten = cfg.defaultGet<bool>("unflatten_reductions", true);
+    recompute = cfg.defaultGet<bool>("recompute_temporaries", true);
     resident = cfg.defaultGet<bool>("resident", true);
     track_host_writes = cfg.defaultGet<bool>("host_write_tracking", true);
     graph_repeats = cfg.defaultGet<bool>("graph_repeats", true);
@@ -823,6 +824,7 @@ void EngineHip::handleExecution(BhIR *bhir) {
     for (bh_base *b : frees) release(b);
     rewrite_store.clear();
     if (unflatten) unflatten_full_reductions(instr_list, rewrite_store);
+    if (recompute) recomputed += static_cast<uint64_t>(recompute_temporaries(instr_list, rewrite_store, bhir->getSyncs()));
     std::vector<TwinUpdate> exchanges;
     if (twin_updates) {
         std::set<bh_base *> syncs;
@@ -859,7 +861,7 @@ void EngineHip::handleExecution(BhIR *bhir) {
         ++flush_cache_misses;
         std::unordered_map<const bh_base *, int> base2ord;  // the flush's base ordinals (inverse of ord2base)
         for (size_t o = 0; o < ord2base.size(); ++o) base2ord.emplace(ord2base[o], static_cast<int>(o));
-        std::vector<jitk::LoopB> kernels = fold_serial_tails(jitk::get_kernel_list(instr_list, fusion_config));
+        std::vector<jitk::LoopB> kernels = fold_row_tails(fold_serial_tails(jitk::get_kernel_list(instr_list, fusion_config)));
         // A kernel releases the bases freed in it when it ends: no later kernel may use them.
         {
             std::set<const bh_base *> released;
@@ -1360,6 +1362,7 @@ std::string EngineHip::statistics() const {
        << "\ntime_finish: " << stats.time_finish << "\n";
     for (const auto &kv : stats.device_ms_by_strategy) ss << "device_ms_" << kv.first << ": " << kv.second << "\n";
     ss << "flush_cache_hits: " << flush_cache_hits << "\nflush_cache_misses: " << flush_cache_misses << "\n";
+    ss << "recomputed: " << recomputed << "\n";
     ss << "missed_frees: " << missed_frees << "\n";
     ss << "buffers: " << bufs.size() << "\nreleases: " << releases << "\n";
     ss << "host_guards: " << host_guards << "\nhost_write_faults: " << g_host_write_faults.load() << "\n";
@@ -1718,6 +1721,8 @@ public:
             engine.track_host_writes = true;
         } else if (msg == "host_write_tracking: off") {
             engine.track_host_writes = false;
+        } else if (msg == "recompute_temporaries: on" || msg == "recompute_temporaries: off") {
+            engine.recompute = msg.back() == 'n';
         } else if (msg == "graph: on") {
             engine.graph_repeats = true;
         } else if (msg == "graph: off") {

@@ -171,12 +171,17 @@ public:
     };
     FlushEffects takeEffects() {
         FlushEffects f;
-        f.written.assign(flush_written.begin(), flush_written.end());
+        // (a base released in the flush has no state left to keep, and a rewrite's own is gone after it)
+        for (bh_base *b : flush_written)
+            if (!released_now.count(b)) f.written.push_back(b);
         f.exchanges.swap(flush_exchanges);
         flush_written.clear();
         return f;
     }
     void applyEffects(const FlushEffects &f);
+    /* Cheap large temporaries are repeated in front of a later reader instead of stored (rewrite.hpp). */
+    bool recompute = true;
+    uint64_t recomputed = 0;
     /* In-place updates through a temporary run as buffer exchanges with a twin (rewrite.hpp). */
     bool twin_updates = true;
     uint64_t twin_min_bytes = 1u << 20;
@@ -196,8 +201,8 @@ public:
 private:
     component::ComponentVE &comp;
     WriterConfig wcfg;
-    bool unflatten = true;       // restate full reductions of N-D temporaries on their shape
     RewriteStore rewrite_store;  // instructions and temporaries added to the current flush
+    bool unflatten = true;       // restate full reductions of N-D temporaries on their shape
     std::string cache_dir;
     bool resident = true;
     int num_cus = 0;  // compute units of the device (0 in compile-only mode)

@@ -1,5 +1,6 @@
 #include "rewrite.hpp"
 
+#include <algorithm>
 #include <map>
 #include <set>
 
@@ -216,6 +217,149 @@ std::vector<TwinUpdate> rewrite_in_place_updates(std::vector<bh_instruction *> &
         }
     }
     return out;
+}
+
+namespace {
+
+// Operations that cost less to repeat than their result costs to store and load again (and that no
+// multiply-add contraction changes when they are repeated next to their reader).
+bool cheap(bh_opcode op) {
+    return op == BH_ADD || op == BH_SUBTRACT || op == BH_MAXIMUM || op == BH_MINIMUM || op == BH_ABSOLUTE ||
+           op == BH_IDENTITY;
+}
+
+// Elements of the base that a view reaches (broadcast axes count once).
+int64_t distinct_elements(const bh_view &v) {
+    int64_t n = 1;
+    for (int64_t d = 0; d < v.ndim; ++d)
+        if (v.stride[d] != 0) n *= v.shape[d];
+    return n;
+}
+
+// Smaller results stay in the caches between the kernels that share them.
+constexpr int64_t kRecomputeBytes = 1 << 20;
+
+} // namespace
+
+int recompute_temporaries(std::vector<bh_instruction *> &list, RewriteStore &store, const std::set<bh_base *> &syncs) {
+    bool sweeps = false;
+    for (const bh_instruction *i : list) {
+        if (i->opcode > BH_MAX_OPCODE_ID) return 0;
+        sweeps |= bh_opcode_is_reduction(i->opcode) != 0;
+    }
+    if (!sweeps) return 0;
+    int count = 0;
+    for (size_t k = 0; k < list.size(); ++k) {
+        const bh_instruction *p = list[k];
+        if (!cheap(p->opcode) || p->operand.size() < 2 || !full_contiguous(p->operand[0])) continue;
+        const bh_view out = p->operand[0];
+        bh_base *T = out.base;
+        if (T->nbytes() < kRecomputeBytes || syncs.count(T)) continue;
+        // Written here only, freed in this flush, read through its whole view only.
+        bool ok = true;
+        size_t freed = kNone;
+        for (size_t j = 0; j < list.size() && ok; ++j) {
+            if (j == k) continue;
+            if (list[j]->opcode == BH_FREE) {
+                if (list[j]->operand[0].base == T) freed = j;
+                continue;
+            }
+            if (!touches(list[j], T)) continue;
+            ok = j > k && !writes(list[j], T);
+            for (size_t o = 1; o < list[j]->operand.size() && ok; ++o) {
+                const bh_view &v = list[j]->operand[o];
+                if (!v.isConstant() && v.base == T) ok = v == out;
+            }
+        }
+        if (!ok || freed == kNone) continue;
+        // One array of T's size at most is read again, and it is not made in this flush (it is in memory).
+        int large = 0;
+        for (size_t o = 1; o < p->operand.size() && ok; ++o) {
+            const bh_view &v = p->operand[o];
+            if (v.isConstant()) continue;
+            ok = v.base != T && !v.hasSlide();
+            if (distinct_elements(v) * 8 > T->nelem()) {
+                ++large;
+                for (const bh_instruction *i : list) ok &= i->opcode == BH_FREE || !writes(i, v.base);
+            }
+        }
+        if (!ok || large > 1) continue;
+        // What follows from T, and the results that follow from a reduction of it.
+        std::set<const bh_base *> from_t{T}, reduced;
+        for (size_t q = k + 1; q < freed; ++q) {
+            const bh_instruction *i = list[q];
+            if (i->opcode == BH_FREE || i->operand.empty() || i->operand[0].isConstant()) continue;
+            bool t = false, r = false, reads_t = false;
+            for (size_t o = 1; o < i->operand.size(); ++o) {
+                const bh_view &v = i->operand[o];
+                if (v.isConstant()) continue;
+                t |= from_t.count(v.base) != 0;
+                r |= reduced.count(v.base) != 0;
+                reads_t |= v.base == T;
+            }
+            if (reads_t && r && !bh_opcode_is_sweep(i->opcode) && i->opcode != BH_GATHER && i->opcode != BH_SCATTER &&
+                i->opcode != BH_COND_SCATTER) {
+                // T's inputs as they were: not written since, and alive (a freed small one lives until q).
+                bool same = true;
+                std::vector<size_t> late;
+                for (size_t o = 1; o < p->operand.size(); ++o) {
+                    const bh_view &v = p->operand[o];
+                    if (v.isConstant()) continue;
+                    for (size_t j = k + 1; j < q; ++j) {
+                        if (list[j]->opcode == BH_FREE) {
+                            if (list[j]->operand[0].base != v.base) continue;
+                            same &= distinct_elements(v) * 8 <= T->nelem();
+                            late.push_back(j);
+                        } else {
+                            same &= !writes(list[j], v.base);
+                        }
+                    }
+                }
+                if (same) {
+                    store.bases.emplace_back(new bh_base(T->nelem(), T->dtype()));
+                    bh_base *again = store.bases.back().get();
+                    store.instrs.push_back(*p);
+                    bh_instruction *made = &store.instrs.back();
+                    made->operand[0].base = again;
+                    store.instrs.push_back(*i);
+                    bh_instruction *reader = &store.instrs.back();
+                    for (size_t o = 1; o < reader->operand.size(); ++o)
+                        if (!reader->operand[o].isConstant() && reader->operand[o].base == T) reader->operand[o].base = again;
+                    store.instrs.push_back(bh_instruction(BH_FREE, {bh_view(again)}));
+                    bh_instruction *fr = &store.instrs.back();
+                    std::vector<bh_instruction *> nl;
+                    nl.reserve(list.size() + 2);
+                    size_t last = k;  // T's last reader: it is freed there
+                    for (size_t j = k + 1; j < list.size(); ++j)
+                        if (j != q && j != freed && touches(list[j], T)) last = j;
+                    for (size_t j = 0; j < list.size(); ++j) {
+                        if (j == freed || std::find(late.begin(), late.end(), j) != late.end()) continue;
+                        if (j == q) nl.push_back(made);
+                        nl.push_back(j == q ? reader : list[j]);
+                        if (j == last) nl.push_back(list[freed]);
+                        if (j == q) {
+                            nl.push_back(fr);
+                            for (size_t f : late) nl.push_back(list[f]);
+                        }
+                    }
+                    // (the lists differ behind k: go on after the reader in the new one)
+                    size_t at = 0;
+                    for (size_t j = 0; j < nl.size(); ++j)
+                        if (nl[j] == reader) at = j;
+                    list.swap(nl);
+                    freed = list.size();
+                    for (size_t j = k + 1; j < list.size(); ++j)
+                        if (list[j]->opcode == BH_FREE && list[j]->operand[0].base == T) freed = j;
+                    i = reader;
+                    q = at;
+                    ++count;
+                }
+            }
+            if (r || (t && bh_opcode_is_reduction(i->opcode))) reduced.insert(i->operand[0].base);
+            if (t) from_t.insert(i->operand[0].base);
+        }
+    }
+    return count;
 }
 
 } // namespace vehip

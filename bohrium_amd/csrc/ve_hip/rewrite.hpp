@@ -37,6 +37,18 @@ struct RewriteStore {
 /* Returns the number of reductions rewritten. */
 int unflatten_full_reductions(std::vector<bh_instruction *> &list, RewriteStore &store);
 
+/* A large temporary that is cheap to compute from at most one array in memory (c = x - m) and that is
+ * read again after something was reduced from it (z = c / s, s from the sum of c * c) cannot stay in a
+ * register: the second reader runs in a later kernel.  Stored, it costs a write and a read of its
+ * size; the rewrite repeats its instruction in front of the later reader instead, which costs one
+ * read of its input.  The same operation on the same values: results do not change.  Conditions: the
+ * temporary is freed in the flush, not synced, written once and read through its whole view; its
+ * inputs are not written between (a small one freed between lives until the later reader).
+ * Measured with the maps folded into the reductions before them (fold_row_tails): column statistics and the
+ * standardised matrix of 100000 x 500 float32 231 -> 176 us, row statistics of 16384 x 3000 198 -> 155 us.
+ * Returns the number of readers rewritten. */
+int recompute_temporaries(std::vector<bh_instruction *> &list, RewriteStore &store, const std::set<bh_base *> &syncs);
+
 /* In-place updates through a temporary, as the front ends emit them for `c[...] = f(views of G)`
  * with c a view of G: T = f(...) (T a temporary of c's shape), IDENTITY(c, T), BH_FREE(T).  Run as
  * written, T makes a round trip through device memory and the copy reads and writes c again.
