@@ -3,6 +3,7 @@
 #include <bohrium/jitk/fuser.hpp>
 
 #include <algorithm>
+#include <cmath>
 #include <functional>
 #include <cstring>
 #include <map>
@@ -46,6 +47,16 @@ const char *hip_type(bh_type t) {
         case bh_type::R123: return "uint64_t";
     }
     throw std::runtime_error("hip_type(): unknown type");
+}
+
+bool divides_by_power_of_two(const bh_instruction &i) {
+    if (i.opcode != BH_DIVIDE || i.operand.size() != 3 || !i.operand[2].isConstant()) return false;
+    int e = 0;
+    if (i.constant.type == bh_type::FLOAT64 && i.operand_type(0) == bh_type::FLOAT64)
+        return std::fabs(std::frexp(i.constant.value.float64, &e)) == 0.5 && std::abs(e - 1) <= 1022;
+    if (i.constant.type == bh_type::FLOAT32 && i.operand_type(0) == bh_type::FLOAT32)
+        return std::fabs(std::frexp(i.constant.value.float32, &e)) == 0.5 && std::abs(e - 1) <= 126;
+    return false;
 }
 
 namespace {
@@ -223,6 +234,11 @@ std::string hip_operation(const bh_instruction &instr, const std::vector<std::st
             if (bh_type_is_signed_integer(instr.operand[0].base->dtype())) {  // NumPy floor division
                 o << a[0] << " = ((" << a[1] << " > 0) != (" << a[2] << " > 0) && (" << a[1] << " % " << a[2]
                   << ") != 0)?(" << a[1] << " / " << a[2] << " - 1):(" << a[1] << " / " << a[2] << ");";
+            } else if (divides_by_power_of_two(instr)) {
+                // x / 2^k is x * 2^-k to the last bit, and the reciprocal leaves the loop (an IEEE float64 division
+                // is 11 instructions, one at a quarter of the rate; every uniform draw divides by 2^64)
+                const char *t = instr.operand_type(0) == bh_type::FLOAT32 ? "float" : "double";
+                o << a[0] << " = " << a[1] << " * ((" << t << ")1 / " << a[2] << ");";
             } else {
                 bin("/");
             }

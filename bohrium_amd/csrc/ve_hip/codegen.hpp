@@ -154,6 +154,10 @@ std::string batch_source(const KernelPlan &plan);
  * level by level with a grid barrier between levels (kernel_prelude bh_grid_sync). */
 std::string persist_source(const std::vector<const KernelPlan *> &codes);
 
+/* A float division by a constant 2^k (either sign) whose reciprocal is a normal number: written as a
+ * multiplication.  The value is an argument, so the plan key says for each such instruction which form it has. */
+bool divides_by_power_of_two(const bh_instruction &i);
+
 /* HIP spelling of an element type inside generated kernels. */
 const char *hip_type(bh_type t);
 

@@ -690,7 +690,7 @@ std::string EngineHip::flushKey(const std::vector<bh_instruction *> &instrs, std
     int64_t nconst = 0;
     for (const bh_instruction *i : instrs) {
         put(i->opcode);
-        put(i->constructor ? 1 : 0);
+        put((i->constructor ? 1 : 0) | (divides_by_power_of_two(*i) ? 2 : 0));
         put(static_cast<int64_t>(i->operand.size()));
         for (const bh_view &v : i->operand) {
             if (v.isConstant()) {
