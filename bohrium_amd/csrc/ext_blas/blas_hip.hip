@@ -2,11 +2,13 @@
  * the reference's blas_* extension methods (include/bh_blas_hip.h).
  *
  * Real types: one workgroup of 4 waves computes a BM x BN tile of C; wave w owns
- * the (w / 2, w % 2) quarter as TM x TN MFMA tiles of 16 x 16.  Per K step (BK
- * of 16 or 32) the workgroup stages op(A) (BM x BK) and op(B) (BK x BN) in LDS
- * with padded rows so that the 16-lane groups of one MFMA operand read fall in
- * disjoint banks; the LDS tiles are double-buffered and the next K step is
- * fetched into registers while the current one runs on the matrix cores.  MFMA operand layout (16 x 16 x 4, measured on gfx950): lane l
+ * the (w / 2, w % 2) quarter as TM x TN MFMA tiles of 16 x 16.  Per K step (16)
+ * the workgroup stages op(A) (BM x BK) and op(B) (BK x BN) in LDS with padded
+ * rows so that the 16-lane groups of one MFMA operand read fall in disjoint
+ * banks; the LDS tiles are double-buffered and the next K step is fetched into
+ * registers while the current one runs on the matrix cores.  Products with too
+ * few such tiles for the chip split K over the waves of a workgroup instead
+ * (gemm_slice).  MFMA operand layout (16 x 16 x 4, measured on gfx950): lane l
  * supplies A[l % 16][l / 16] and B[l / 16][l % 16]; its 4 results are
  * D[4 (l / 16) + r][l % 16] for f32 and D[4 r + l / 16][l % 16] for f64, r = 0..3.
  *
@@ -16,7 +18,6 @@
 
 #include <algorithm>
 #include <cstdint>
-#include <cstdlib>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -52,22 +53,31 @@ template <> struct Mfma<float> {
 constexpr int kThreads = 256;
 constexpr int kPad = 16;
 
+// 16 bytes of elements; `loose`: at any element (a global load needs no more than 4-byte alignment).
 template <typename T> struct Vec;
 template <> struct Vec<double> {
     typedef double type __attribute__((ext_vector_type(2)));
+    typedef double loose __attribute__((ext_vector_type(2), aligned(8)));
     static constexpr int n = 2;
 };
 template <> struct Vec<float> {
     typedef float type __attribute__((ext_vector_type(4)));
+    typedef float loose __attribute__((ext_vector_type(4), aligned(4)));
     static constexpr int n = 4;
 };
 
-// One operand tile: ROWS rows (m of op(A) or n of op(B)) by kBK steps of k (16 or 32).  KCONT: k is the
-// contiguous dimension in memory (element (r, k) at P[r * ld + k]); otherwise r is
-// (element at P[k * ld + r]).  A thread moves chunks of V elements along the contiguous dimension
-// (one 16-byte load on interior tiles).  LDS layout: [ROWS][kBK + KPAD] when KCONT, else
-// [kBK][ROWS + kPad]; with these pads the 16-lane groups of an MFMA operand read (16 rows at one k,
-// the next group at k + 1) and the chunk stores fall in disjoint banks.
+// One operand tile: ROWS rows (m of op(A) or n of op(B)) by kBK steps of k.  KCONT: k is the contiguous
+// dimension in memory (element (r, k) at P[r * ld + k]); otherwise r is (element at P[k * ld + r]).  A thread
+// moves CH chunks of V elements along the contiguous dimension, one 16-byte load each at any alignment.
+// LDS layout: [ROWS][kBK + KPAD] when KCONT, else [kBK][ROWS + kPad]; with these pads the 16-lane groups of
+// an MFMA operand read (16 rows at one k, the next group at k + 1) and the chunk stores fall in disjoint
+// banks.
+//
+// The loads of the main loop have no bounds checks (a check is a branch, and the compiler waits for the
+// loads at its join: the prefetch of the next K step was not overlapped at all).  Rows past R are taken
+// from inside the matrix instead, their results are not stored: KCONT chunks repeat row R - 1; the others
+// move down to end at row R - 1, in LDS too (`edge`: stored element by element).  Needs R >= V.  The K % kBK
+// leading columns are a step of their own (`first`), zero-filled.
 template <typename T, bool KCONT, int ROWS, int kBK>
 struct Tile {
     static constexpr int V = Vec<T>::n;
@@ -76,8 +86,14 @@ struct Tile {
     static constexpr int KPAD = sizeof(T) == 8 ? 2 : 4;
     static constexpr int LDS = KCONT ? ROWS * (kBK + KPAD) : kBK * (ROWS + kPad);
     static_assert(CH * V == PER && CH * kThreads * V == ROWS * kBK, "tile / thread count");
+    typedef typename Vec<T>::loose Loose;
 
-    static __device__ __forceinline__ void chunk(int c, int &r, int &k) {
+    const T *p[CH];  // the chunks of the next step
+    int64_t advance;
+    T reg[PER];
+
+    static __device__ __forceinline__ void chunk(int e, int &r, int &k) {
+        const int c = static_cast<int>(threadIdx.x) + e * kThreads;
         if (KCONT) {
             r = c / (kBK / V);
             k = (c % (kBK / V)) * V;
@@ -86,33 +102,46 @@ struct Tile {
             r = (c % (ROWS / V)) * V;
         }
     }
-    // vec: the whole tile is in bounds and every chunk is 16-byte aligned.
-    static __device__ __forceinline__ void fetch(const T *__restrict__ P, int64_t ld, int64_t r0, int64_t k0, int64_t R,
-                                                 int64_t K, bool vec, T *reg) {
+    // The row that chunk (r) of a tile at r0 is loaded from.
+    static __device__ __forceinline__ int64_t source(int64_t r0, int r, int64_t R) {
+        const int64_t last = KCONT ? R - 1 : R - V;
+        return r0 + r < last ? r0 + r : last;
+    }
+    // Loads columns [0, kn) of the tile (kn <= kBK, zeros past it) and points at column kn.
+    __device__ __forceinline__ void first(const T *__restrict__ P, int64_t ld, int64_t r0, int64_t R, int kn) {
+        advance = KCONT ? kBK : kBK * ld;
 #pragma unroll
         for (int e = 0; e < CH; ++e) {
             int r, k;
-            chunk(static_cast<int>(threadIdx.x) + e * kThreads, r, k);
-            const int64_t gr = r0 + r, gk = k0 + k;
-            if (vec) {
-                const typename Vec<T>::type v =
-                    *reinterpret_cast<const typename Vec<T>::type *>(KCONT ? P + gr * ld + gk : P + gk * ld + gr);
+            chunk(e, r, k);
+            const int64_t gr = source(r0, r, R);
+            const T *q = KCONT ? P + gr * ld + k : P + k * ld + gr;
 #pragma unroll
-                for (int j = 0; j < V; ++j) reg[e * V + j] = v[j];
-            } else {
-#pragma unroll
-                for (int j = 0; j < V; ++j) {
-                    const int64_t rr = KCONT ? gr : gr + j, kk = KCONT ? gk + j : gk;
-                    reg[e * V + j] = (rr < R && kk < K) ? P[KCONT ? rr * ld + kk : kk * ld + rr] : T(0);
-                }
-            }
+            for (int j = 0; j < V; ++j) reg[e * V + j] = (KCONT ? k + j : k) < kn ? q[j] : T(0);
+            p[e] = q + (KCONT ? kn : kn * ld);
         }
     }
-    static __device__ __forceinline__ void store(T *lds, const T *reg) {
+    __device__ __forceinline__ void next() {
+#pragma unroll
+        for (int e = 0; e < CH; ++e) {
+            const Loose v = *reinterpret_cast<const Loose *>(p[e]);
+            p[e] += advance;
+#pragma unroll
+            for (int j = 0; j < V; ++j) reg[e * V + j] = v[j];
+        }
+    }
+    __device__ __forceinline__ void store(T *lds, bool edge, int64_t r0, int64_t R) const {
 #pragma unroll
         for (int e = 0; e < CH; ++e) {
             int r, k;
-            chunk(static_cast<int>(threadIdx.x) + e * kThreads, r, k);
+            chunk(e, r, k);
+            if (!KCONT && edge) {
+                const int at = static_cast<int>(source(r0, r, R) - r0);
+#pragma unroll
+                for (int j = 0; j < V; ++j)
+                    if (at + j >= 0) lds[k * (ROWS + kPad) + at + j] = reg[e * V + j];
+                continue;
+            }
             typename Vec<T>::type v;
 #pragma unroll
             for (int j = 0; j < V; ++j) v[j] = reg[e * V + j];
@@ -128,13 +157,16 @@ struct Tile {
 // = TA ? A[k * lda + m] : A[m * lda + k], op(B)(k, n) = TB ? B[n * ldb + k] : B[k * ldb + n].  UPPER:
 // only C(m, n) with m <= n is stored.  The scaled epilogue is a separate instantiation: in the plain
 // product it costs the f64 128 x 128 kernel ~120 VGPRs and half its throughput.
-// vec_ok: lda and ldb are multiples of the 16-byte vector and A, B are 16-byte aligned.
 // The LDS tiles are double-buffered: while the matrix cores work on one K step, the next one is
-// loaded into registers and then stored into the other buffer; one barrier per K step.
+// loaded into registers and then stored into the other buffer; one barrier per K step.  Two waves a SIMD: the
+// epilogue alone would take the f64 128 x 128 kernel to 278 registers and one wave.
+// Bound by the MFMA rate (counters: the matrix cores were busy 76 % of the cycles while the loads waited at
+// bounds checks).  Measured with the checks out of the loop: 4096^3 f64 2364 -> 2078 us (66.1 TFLOP/s; the
+// library 66-69), f32 1118 -> 1029 us; 2000 x 1500 x 2500 f64 344 -> 267 us, f32 189 -> 155 us.
 template <typename T, bool TA, bool TB, bool UPPER, int TM, int TN, int BK, bool SCALED>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kThreads, 2)
 gemm_mfma(const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C, int64_t M, int64_t N, int64_t K,
-          int64_t lda, int64_t ldb, int64_t ldc, int vec_ok, T alpha, T beta) {
+          int64_t lda, int64_t ldb, int64_t ldc, T alpha, T beta) {
     constexpr int BM = 32 * TM, BN = 32 * TN;
     typedef Tile<T, !TA, BM, BK> ATile;
     typedef Tile<T, TB, BN, BK> BTile;
@@ -145,7 +177,7 @@ gemm_mfma(const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C, i
     const int64_t bm = static_cast<int64_t>(blockIdx.y) * BM, bn = static_cast<int64_t>(blockIdx.x) * BN;
     if (UPPER && bm > bn + BN - 1) return;  // the whole tile lies below the diagonal
     const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
-    const bool a_in = vec_ok && bm + BM <= M, b_in = vec_ok && bn + BN <= N;
+    const bool a_edge = bm + BM > M, b_edge = bn + BN > N;
 
     typename Mfma<T>::Acc acc[TM][TN];
 #pragma unroll
@@ -155,21 +187,7 @@ gemm_mfma(const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C, i
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[i][j][r] = T(0);
 
-    T ra[ATile::PER], rb[BTile::PER];
-    auto fetch = [&](int64_t k0) {
-        const bool kin = k0 + BK <= K;
-        ATile::fetch(A, lda, bm, k0, M, K, a_in && kin, ra);
-        BTile::fetch(B, ldb, bn, k0, N, K, b_in && kin, rb);
-    };
-
-    fetch(0);
-    ATile::store(As[0], ra);
-    BTile::store(Bs[0], rb);
-    __syncthreads();
-    int buf = 0;
-    for (int64_t k0 = 0; k0 < K; k0 += BK) {
-        const bool more = k0 + BK < K;
-        if (more) fetch(k0 + BK);
+    auto multiply = [&](int buf) {
         const T *as = As[buf], *bs = Bs[buf];
 #pragma unroll
         for (int ks = 0; ks < BK; ks += 4) {
@@ -184,13 +202,28 @@ gemm_mfma(const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C, i
 #pragma unroll
                 for (int j = 0; j < TN; ++j) acc[i][j] = Mfma<T>::step(a[i], b[j], acc[i][j]);
         }
-        if (more) {
-            ATile::store(As[buf ^ 1], ra);
-            BTile::store(Bs[buf ^ 1], rb);
-        }
-        // the other buffer is complete, and every wave is done reading this one before it is refilled
+    };
+    ATile ta;
+    BTile tb;
+    if (K > 0) {
+        const int kn = K % BK != 0 ? static_cast<int>(K % BK) : BK;
+        ta.first(A, lda, bm, M, kn);
+        tb.first(B, ldb, bn, N, kn);
+        ta.store(As[0], a_edge, bm, M);
+        tb.store(Bs[0], b_edge, bn, N);
         __syncthreads();
-        buf ^= 1;
+        int buf = 0;
+        for (int64_t k = kn; k < K; k += BK) {
+            ta.next();
+            tb.next();
+            multiply(buf);
+            buf ^= 1;
+            ta.store(As[buf], a_edge, bm, M);
+            tb.store(Bs[buf], b_edge, bn, N);
+            // the buffer is complete, and every wave is done reading the other before it is refilled
+            __syncthreads();
+        }
+        multiply(buf);
     }
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -240,7 +273,7 @@ template <typename R> __device__ __forceinline__ Cplx<R> msub(Cplx<R> s, Cplx<R>
 // buffering as in gemm_mfma; the LDS rows are padded to an odd number of 16-byte elements (c128) or to two
 // 8-byte elements more than a multiple of 16 (c64), so the 16-lane groups of a read fall in disjoint banks.
 // Measured against one FMA thread per element of C: 4096^3 c128 22.8 -> 65.2 TFLOP/s (24.1 -> 8.4 ms), c64
-// 34.6 -> 121 TFLOP/s; 2000 x 1500 x 2500 c128 2678 -> 984 us, 256^3 14.4 -> 14.8 us.
+// 34.6 -> 121 TFLOP/s; 2000 x 1500 x 2500 c128 2678 -> 984 us, with the bounds checks out of the loop 901 us.
 template <typename R, bool KCONT, int ROWS, int kBK>
 struct CTile {
     static constexpr int CH = ROWS * kBK / kThreads;
@@ -249,22 +282,36 @@ struct CTile {
     static constexpr int LDS = KCONT ? ROWS * (kBK + KPAD) : kBK * (ROWS + RPAD);
     static_assert(CH * kThreads == ROWS * kBK, "tile / thread count");
 
+    const Cplx<R> *p[CH];  // the elements of the next step
+    int64_t advance;
+    Cplx<R> reg[CH];
+
     static __device__ __forceinline__ void place(int e, int &r, int &k) {
         const int c = static_cast<int>(threadIdx.x) + e * kThreads;
         r = KCONT ? c / kBK : c % ROWS;
         k = KCONT ? c % kBK : c / ROWS;
     }
-    static __device__ __forceinline__ void fetch(const Cplx<R> *__restrict__ P, int64_t ld, int64_t r0, int64_t k0,
-                                                 int64_t Rn, int64_t K, Cplx<R> *reg) {
+    // As Tile::first and next; rows past Rn repeat row Rn - 1.
+    __device__ __forceinline__ void first(const Cplx<R> *__restrict__ P, int64_t ld, int64_t r0, int64_t Rn, int kn) {
+        advance = KCONT ? kBK : kBK * ld;
 #pragma unroll
         for (int e = 0; e < CH; ++e) {
             int r, k;
             place(e, r, k);
-            const int64_t gr = r0 + r, gk = k0 + k;
-            reg[e] = gr < Rn && gk < K ? P[KCONT ? gr * ld + gk : gk * ld + gr] : Cplx<R>{R(0), R(0)};
+            const int64_t gr = r0 + r < Rn ? r0 + r : Rn - 1;
+            const Cplx<R> *q = KCONT ? P + gr * ld + k : P + k * ld + gr;
+            reg[e] = k < kn ? *q : Cplx<R>{R(0), R(0)};
+            p[e] = q + (KCONT ? kn : kn * ld);
         }
     }
-    static __device__ __forceinline__ void store(Cplx<R> *lds, const Cplx<R> *reg) {
+    __device__ __forceinline__ void next() {
+#pragma unroll
+        for (int e = 0; e < CH; ++e) {
+            reg[e] = *p[e];
+            p[e] += advance;
+        }
+    }
+    __device__ __forceinline__ void store(Cplx<R> *lds) const {
 #pragma unroll
         for (int e = 0; e < CH; ++e) {
             int r, k;
@@ -278,7 +325,7 @@ struct CTile {
 };
 
 template <typename R, bool TA, bool TB, bool CONJB, bool UPPER, bool REALDIAG, bool SCALED, int TM, int TN, int BK>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kThreads, 2)
 gemm_complex(const Cplx<R> *__restrict__ A, const Cplx<R> *__restrict__ B, Cplx<R> *__restrict__ C, int64_t M,
              int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, R alpha, R beta) {
     constexpr int BM = 32 * TM, BN = 32 * TN;
@@ -297,19 +344,7 @@ gemm_complex(const Cplx<R> *__restrict__ A, const Cplx<R> *__restrict__ B, Cplx<
         for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) re[i][j][r] = im[i][j][r] = R(0);
-    Cplx<R> ra[ATile::CH], rb[BTile::CH];
-    auto fetch = [&](int64_t k0) {
-        ATile::fetch(A, lda, bm, k0, M, K, ra);
-        BTile::fetch(B, ldb, bn, k0, N, K, rb);
-    };
-    fetch(0);
-    ATile::store(As[0], ra);
-    BTile::store(Bs[0], rb);
-    __syncthreads();
-    int buf = 0;
-    for (int64_t k0 = 0; k0 < K; k0 += BK) {
-        const bool more = k0 + BK < K;
-        if (more) fetch(k0 + BK);
+    auto multiply = [&](int buf) {
         const Cplx<R> *as = As[buf], *bs = Bs[buf];
 #pragma unroll
         for (int ks = 0; ks < BK; ks += 4) {
@@ -334,13 +369,28 @@ gemm_complex(const Cplx<R> *__restrict__ A, const Cplx<R> *__restrict__ B, Cplx<
                 }
             }
         }
-        if (more) {
-            ATile::store(As[buf ^ 1], ra);
-            BTile::store(Bs[buf ^ 1], rb);
-        }
-        // the other buffer is complete, and every wave is done reading this one before it is refilled
+    };
+    ATile ta;
+    BTile tb;
+    if (K > 0) {
+        const int kn = K % BK != 0 ? static_cast<int>(K % BK) : BK;
+        ta.first(A, lda, bm, M, kn);
+        tb.first(B, ldb, bn, N, kn);
+        ta.store(As[0]);
+        tb.store(Bs[0]);
         __syncthreads();
-        buf ^= 1;
+        int buf = 0;
+        for (int64_t k = kn; k < K; k += BK) {
+            ta.next();
+            tb.next();
+            multiply(buf);
+            buf ^= 1;
+            ta.store(As[buf]);
+            tb.store(Bs[buf]);
+            // the buffer is complete, and every wave is done reading the other before it is refilled
+            __syncthreads();
+        }
+        multiply(buf);
     }
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -364,6 +414,159 @@ gemm_complex(const Cplx<R> *__restrict__ A, const Cplx<R> *__restrict__ B, Cplx<
                     if (REALDIAG && row == col) v.im = 0;
                     C[row * ldc + col] = v;
                 }
+            }
+}
+
+// ---- small products: K split over the waves of a workgroup.  A product with few tiles leaves most CUs idle
+// in the kernels above (100 x 100 x 4000: 4 workgroups), and each of its tiles is one serial chain over
+// K.  Here a workgroup computes a 16 TM x 16 TN tile with WAVES waves, wave w the K steps w, w + WAVES, ...
+// of 16, straight from global memory (no sharing to stage for; a lane loads 4 neighbouring k where K is
+// contiguous), and the partial tiles are folded through LDS in a fixed order.  Measured: 100 x 100 x 4000 f64
+// 323 -> 24 us, f32 204 -> 12, c128 292 -> 43; 512^3 f64 30 -> 11; 256^3 f64 16 -> 4.4, c128 14.4 -> 6.4;
+// 2048 x 64 x 2048 f32 67 -> 13 us.
+template <typename E> struct Prod {
+    typedef typename Mfma<E>::Acc Acc;
+    typedef E Real;
+    static __device__ __forceinline__ E zero() { return E(0); }
+    static __device__ __forceinline__ void clear(Acc &c) { c = Acc{}; }
+    static __device__ __forceinline__ void step(E a, E b, Acc &c) { c = Mfma<E>::step(a, b, c); }
+    static __device__ __forceinline__ void add(Acc &c, const Acc &d) { c += d; }
+    static __device__ __forceinline__ E get(const Acc &c, int r) { return c[r]; }
+    static __device__ __forceinline__ int row(int lane, int r) { return Mfma<E>::row(lane, r); }
+    static __device__ __forceinline__ E scaled(E v, E alpha, E beta, const E *old) {
+        v *= alpha;
+        return beta != E(0) ? v + beta * *old : v;
+    }
+    static __device__ __forceinline__ E real_diagonal(E v) { return v; }
+};
+template <typename R> struct Prod<Cplx<R> > {
+    typedef Cplx<R> E;
+    typedef R Real;
+    struct Acc {
+        typename Mfma<R>::Acc re, im;
+    };
+    static __device__ __forceinline__ E zero() { return E{R(0), R(0)}; }
+    static __device__ __forceinline__ void clear(Acc &c) { c.re = c.im = typename Mfma<R>::Acc{}; }
+    static __device__ __forceinline__ void step(E a, E b, Acc &c) {
+        c.re = Mfma<R>::step(a.re, b.re, c.re);
+        c.im = Mfma<R>::step(a.re, b.im, c.im);
+        c.re = Mfma<R>::step(-a.im, b.im, c.re);
+        c.im = Mfma<R>::step(a.im, b.re, c.im);
+    }
+    static __device__ __forceinline__ void add(Acc &c, const Acc &d) {
+        c.re += d.re;
+        c.im += d.im;
+    }
+    static __device__ __forceinline__ E get(const Acc &c, int r) { return E{c.re[r], c.im[r]}; }
+    static __device__ __forceinline__ int row(int lane, int r) { return Mfma<R>::row(lane, r); }
+    static __device__ __forceinline__ E scaled(E v, R alpha, R beta, const E *old) {
+        v.re *= alpha;
+        v.im *= alpha;
+        if (beta != R(0)) {
+            v.re = fma(beta, old->re, v.re);
+            v.im = fma(beta, old->im, v.im);
+        }
+        return v;
+    }
+    static __device__ __forceinline__ E real_diagonal(E v) { return E{v.re, R(0)}; }
+};
+
+template <typename E, bool TA, bool TB, bool CONJB, bool UPPER, bool REALDIAG, bool SCALED, int TM, int TN, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES)
+gemm_slice(const E *__restrict__ A, const E *__restrict__ B, E *__restrict__ C, int64_t M, int64_t N, int64_t K,
+           int64_t lda, int64_t ldb, int64_t ldc, typename Prod<E>::Real alpha, typename Prod<E>::Real beta) {
+    typedef Prod<E> P;
+    constexpr int BM = 16 * TM, BN = 16 * TN, KC = 16;
+    __shared__ __attribute__((aligned(16))) typename P::Acc part[WAVES > 1 ? WAVES / 2 : 1][TM * TN][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t bm = static_cast<int64_t>(blockIdx.y) * BM, bn = static_cast<int64_t>(blockIdx.x) * BN;
+    if (UPPER && bm > bn + BN - 1) return;  // the whole tile lies below the diagonal
+    typename P::Acc acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) P::clear(acc[i][j]);
+    // rows and columns past the edges repeat the last one: their results are not stored
+    int64_t row[TM], col[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) row[i] = bm + i * 16 + (lane & 15) < M ? bm + i * 16 + (lane & 15) : M - 1;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) col[j] = bn + j * 16 + (lane & 15) < N ? bn + j * 16 + (lane & 15) : N - 1;
+    const int q = (lane >> 4) * 4;
+    E a[2][TM][4], b[2][TN][4];
+    auto load = [&](int64_t k0, int w) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int64_t k = k0 + q + s;
+            const bool in = k < K;
+#pragma unroll
+            for (int i = 0; i < TM; ++i) a[w][i][s] = in ? (TA ? A[k * lda + row[i]] : A[row[i] * lda + k]) : P::zero();
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                E v = in ? (TB ? B[col[j] * ldb + k] : B[k * ldb + col[j]]) : P::zero();
+                b[w][j][s] = CONJB ? conj_of(v) : v;
+            }
+        }
+    };
+    auto load_in = [&](int64_t k0, int w) {  // a whole step: no bounds checks
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int64_t k = k0 + q + s;
+#pragma unroll
+            for (int i = 0; i < TM; ++i) a[w][i][s] = TA ? A[k * lda + row[i]] : A[row[i] * lda + k];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const E v = TB ? B[col[j] * ldb + k] : B[k * ldb + col[j]];
+                b[w][j][s] = CONJB ? conj_of(v) : v;
+            }
+        }
+    };
+    auto multiply = [&](int w) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) P::step(a[w][i][s], b[w][j][s], acc[i][j]);
+    };
+    const int64_t whole = K / KC;  // steps of 16 without a remainder
+    int64_t c = wave;
+    if (c < whole) load_in(c * KC, 0);
+    for (; c + WAVES < whole; c += 2 * WAVES) {  // two steps a round, the next one loaded while one is multiplied
+        load_in((c + WAVES) * KC, 1);
+        multiply(0);
+        if (c + 2 * WAVES < whole) load_in((c + 2 * WAVES) * KC, 0);
+        multiply(1);
+    }
+    if (c < whole) multiply(0);
+    if (whole * KC < K && wave == static_cast<int>(whole % WAVES)) {
+        load(whole * KC, 0);
+        multiply(0);
+    }
+#pragma unroll
+    for (int h = WAVES / 2; h >= 1; h /= 2) {
+        if (wave >= h && wave < 2 * h)
+#pragma unroll
+            for (int t = 0; t < TM * TN; ++t) part[wave - h][t][lane] = acc[t / TN][t % TN];
+        __syncthreads();
+        if (wave < h)
+#pragma unroll
+            for (int t = 0; t < TM * TN; ++t) P::add(acc[t / TN][t % TN], part[wave][t][lane]);
+        __syncthreads();
+    }
+    if (wave != 0) return;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int64_t m = bm + i * 16 + P::row(lane, r), n = bn + j * 16 + (lane & 15);
+                if (m >= M || n >= N || (UPPER && m > n)) continue;
+                E v = P::get(acc[i][j], r);
+                if (SCALED) v = P::scaled(v, alpha, beta, C + m * ldc + n);
+                if (REALDIAG && m == n) v = P::real_diagonal(v);
+                C[m * ldc + n] = v;
             }
 }
 
@@ -434,48 +637,62 @@ struct Gemm {
     hipStream_t s;
 };
 
+int64_t tiles(const Gemm &g, int64_t bm, int64_t bn) { return ((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn); }
+
+// The 256 CUs need a workgroup each: fewer 64 x 64 tiles than that, and K is split over waves instead
+// (gemm_slice), with the largest tile that still gives 256 workgroups.  Measured, tile / slice: 1001 x 777 x
+// 1303 (208 tiles) f64 69 / 63 us, f32 75 / 40, c128 188 / 205, c64 122 / 105; 512^3 (64 tiles) f64 26 / 11,
+// f32 18 / 7, c128 74 / 26, c64 47 / 15; 2000 x 1500 x 2500 (768 tiles) f64 267 / 352, f32 155 / 209.
+// (The tiles' chunks need as many rows and columns as a vector has elements.)
+constexpr int64_t kFill = 256;
+bool use_tiles(const Gemm &g) { return tiles(g, 64, 64) >= kFill && g.m >= 16 && g.n >= 16; }
+
+template <typename E, bool TA, bool TB, bool CONJB, bool UPPER, bool REALDIAG, bool SCALED, int TM, int TN, int WAVES>
+void launch_slice_tile(const Gemm &g) {
+    typedef typename Prod<E>::Real R;
+    const dim3 grid(static_cast<unsigned>((g.n + 16 * TN - 1) / (16 * TN)),
+                    static_cast<unsigned>((g.m + 16 * TM - 1) / (16 * TM)));
+    gemm_slice<E, TA, TB, CONJB, UPPER, REALDIAG, SCALED, TM, TN, WAVES><<<grid, 64 * WAVES, 0, g.s>>>(
+        static_cast<const E *>(g.A), static_cast<const E *>(g.B), static_cast<E *>(g.C), g.m, g.n, g.k, g.lda, g.ldb,
+        g.ldc, static_cast<R>(g.alpha), static_cast<R>(g.beta));
+}
+
+template <typename E, bool TA, bool TB, bool CONJB, bool UPPER, bool REALDIAG, bool SCALED>
+void launch_slice(const Gemm &g) {
+    if (tiles(g, 32, 32) >= kFill)
+        launch_slice_tile<E, TA, TB, CONJB, UPPER, REALDIAG, SCALED, 2, 2, 4>(g);
+    else if (sizeof(E) == sizeof(typename Prod<E>::Real) && tiles(g, 16, 32) >= kFill)
+        launch_slice_tile<E, TA, TB, CONJB, UPPER, REALDIAG, SCALED, 1, 2, 8>(g);
+    else
+        launch_slice_tile<E, TA, TB, CONJB, UPPER, REALDIAG, SCALED, 1, 1, 8>(g);
+}
+
+template <typename T, bool TA, bool TB, bool UPPER, bool SCALED, int TM>
+void launch_real_tile(const Gemm &g) {
+    const dim3 grid(static_cast<unsigned>((g.n + 32 * TM - 1) / (32 * TM)),
+                    static_cast<unsigned>((g.m + 32 * TM - 1) / (32 * TM)));
+    gemm_mfma<T, TA, TB, UPPER, TM, TM, 16, SCALED><<<grid, kThreads, 0, g.s>>>(
+        static_cast<const T *>(g.A), static_cast<const T *>(g.B), static_cast<T *>(g.C), g.m, g.n, g.k, g.lda, g.ldb,
+        g.ldc, static_cast<T>(g.alpha), static_cast<T>(g.beta));
+}
+
 template <typename T, bool TA, bool TB, bool UPPER, bool SCALED>
-void launch_real_tiles(const Gemm &g, int vec_ok) {
-    // 128 x 128 tiles when the matrix fills the device with them, 64 x 64 otherwise; K steps of
-    // BH_BLAS_BK elements (16 or 32; 16 measured faster on MI355X: 8192^3 fp64 59.5 vs 40.6,
-    // fp32 129.1 vs 120.0 TFLOP/s).
-    static const int bk = [] {
-        const char *e = std::getenv("BH_BLAS_BK");
-        return e != nullptr && std::atoi(e) == 32 ? 32 : 16;
-    }();
-    const int64_t m = g.m, n = g.n;
-    const bool big = ((m + 127) / 128) * ((n + 127) / 128) >= 512;
-    const T *a = static_cast<const T *>(g.A), *b = static_cast<const T *>(g.B);
-    T *c = static_cast<T *>(g.C);
-    const T al = static_cast<T>(g.alpha), be = static_cast<T>(g.beta);
-    if (big) {
-        const dim3 grid(static_cast<unsigned>((n + 127) / 128), static_cast<unsigned>((m + 127) / 128));
-        if (bk == 32)
-            gemm_mfma<T, TA, TB, UPPER, 4, 4, 32, SCALED>
-                <<<grid, kThreads, 0, g.s>>>(a, b, c, m, n, g.k, g.lda, g.ldb, g.ldc, vec_ok, al, be);
-        else
-            gemm_mfma<T, TA, TB, UPPER, 4, 4, 16, SCALED>
-                <<<grid, kThreads, 0, g.s>>>(a, b, c, m, n, g.k, g.lda, g.ldb, g.ldc, vec_ok, al, be);
-    } else {
-        const dim3 grid(static_cast<unsigned>((n + 63) / 64), static_cast<unsigned>((m + 63) / 64));
-        if (bk == 32)
-            gemm_mfma<T, TA, TB, UPPER, 2, 2, 32, SCALED>
-                <<<grid, kThreads, 0, g.s>>>(a, b, c, m, n, g.k, g.lda, g.ldb, g.ldc, vec_ok, al, be);
-        else
-            gemm_mfma<T, TA, TB, UPPER, 2, 2, 16, SCALED>
-                <<<grid, kThreads, 0, g.s>>>(a, b, c, m, n, g.k, g.lda, g.ldb, g.ldc, vec_ok, al, be);
-    }
+void launch_real_scaled(const Gemm &g) {
+    // 128 x 128 tiles when the matrix gives every CU two workgroups of them, else 64 x 64
+    if (!use_tiles(g))
+        launch_slice<T, TA, TB, false, UPPER, false, SCALED>(g);
+    else if (tiles(g, 128, 128) >= 2 * kFill)
+        launch_real_tile<T, TA, TB, UPPER, SCALED, 4>(g);
+    else
+        launch_real_tile<T, TA, TB, UPPER, SCALED, 2>(g);
 }
 
 template <typename T, bool TA, bool TB, bool UPPER>
 bool launch_real(const Gemm &g) {
-    const int64_t v = Vec<T>::n;
-    const int vec_ok = g.lda % v == 0 && g.ldb % v == 0 && reinterpret_cast<uintptr_t>(g.A) % 16 == 0 &&
-                       reinterpret_cast<uintptr_t>(g.B) % 16 == 0;
     if (g.alpha == 1.0 && g.beta == 0.0) {
-        launch_real_tiles<T, TA, TB, UPPER, false>(g, vec_ok);
+        launch_real_scaled<T, TA, TB, UPPER, false>(g);
     } else if constexpr (!TA) {  // trsm's updates and syr2k's second pass
-        launch_real_tiles<T, TA, TB, UPPER, true>(g, vec_ok);
+        launch_real_scaled<T, TA, TB, UPPER, true>(g);
     } else {
         g_err = "bhblas: scaled product with a transposed A is not provided";
         return false;
@@ -483,22 +700,17 @@ bool launch_real(const Gemm &g) {
     return true;
 }
 
-template <typename R, bool TA, bool TB, bool CONJB, bool UPPER, bool REALDIAG, bool SCALED, int TM, int TN, int BK>
-void launch_complex_tiles(const Gemm &g) {
-    const dim3 grid(static_cast<unsigned>((g.n + 32 * TN - 1) / (32 * TN)),
-                    static_cast<unsigned>((g.m + 32 * TM - 1) / (32 * TM)));
-    gemm_complex<R, TA, TB, CONJB, UPPER, REALDIAG, SCALED, TM, TN, BK><<<grid, kThreads, 0, g.s>>>(
-        static_cast<const Cplx<R> *>(g.A), static_cast<const Cplx<R> *>(g.B), static_cast<Cplx<R> *>(g.C), g.m, g.n,
-        g.k, g.lda, g.ldb, g.ldc, static_cast<R>(g.alpha), static_cast<R>(g.beta));
-}
-
 template <typename R, bool TA, bool TB, bool CONJB, bool UPPER, bool REALDIAG, bool SCALED>
 void launch_complex_scaled(const Gemm &g) {
-    // 64 x 64 tiles when there is a workgroup of them for each of the 256 CUs, else 32 x 32
-    if (((g.m + 63) / 64) * ((g.n + 63) / 64) >= 256)
-        launch_complex_tiles<R, TA, TB, CONJB, UPPER, REALDIAG, SCALED, 2, 2, sizeof(R) == 8 ? 8 : 16>(g);
-    else
-        launch_complex_tiles<R, TA, TB, CONJB, UPPER, REALDIAG, SCALED, 1, 1, 16>(g);
+    if (!use_tiles(g)) {
+        launch_slice<Cplx<R>, TA, TB, CONJB, UPPER, REALDIAG, SCALED>(g);
+        return;
+    }
+    constexpr int BK = sizeof(R) == 8 ? 8 : 16;
+    const dim3 grid(static_cast<unsigned>((g.n + 63) / 64), static_cast<unsigned>((g.m + 63) / 64));
+    gemm_complex<R, TA, TB, CONJB, UPPER, REALDIAG, SCALED, 2, 2, BK><<<grid, kThreads, 0, g.s>>>(
+        static_cast<const Cplx<R> *>(g.A), static_cast<const Cplx<R> *>(g.B), static_cast<Cplx<R> *>(g.C), g.m, g.n,
+        g.k, g.lda, g.ldb, g.ldc, static_cast<R>(g.alpha), static_cast<R>(g.beta));
 }
 
 template <typename R, bool TA, bool TB, bool CONJB, bool UPPER, bool REALDIAG>

@@ -357,3 +357,38 @@ def test_gemm_inside_a_repeated_body():
     mag = np.abs(a) @ (np.abs(a) @ (np.abs(a) @ np.abs(x0)))
     assert np.all(np.abs(got - want) <= 3 * 64 * 2.0 ** -53 * mag + 1e-300)
     assert not np.allclose(got, a @ x0)  # more than one iteration ran
+
+
+# One element below, at and above a tile, a vector, a K step and a wave's share, for each kernel that the sizes
+# choose: K split over 4 and 8 waves (tiles of 32 x 32, 16 x 32, 16 x 16), 64 x 64 and 128 x 128 tiles.
+EDGES = [(1, 3, 1), (3, 1, 700), (15, 17, 129), (17, 33, 16), (100, 100, 1001), (250, 270, 63), (500, 600, 65),
+         (1030, 1021, 67), (1023, 1090, 8), (16385, 17, 31), (17, 16385, 9), (16500, 3, 40), (3000, 2945, 33)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.complex128, np.complex64])
+@pytest.mark.parametrize("m,n,k", EDGES)
+def test_gemm_edges(dtype, m, n, k):
+    import bohrium_amd as bh
+    a, b = _rand((m, k), dtype, 1), _rand((k, n), dtype, 2)
+    # NaN around the operands in memory: no result may depend on what lies outside them
+    A, B = bh.array(np.full((m + 2, k), np.nan, dtype)), bh.array(np.full((k + 2, n), np.nan, dtype))
+    A[1:-1], B[1:-1] = bh.array(a), bh.array(b)
+    bh.flush()
+    _check(bh.blas.gemm(A[1:-1], B[1:-1]).asnumpy(), a, b, dtype)
+    if m * k < 2 ** 21:
+        at = np.ascontiguousarray(a.T)
+        _check(bh.blas.gemmt(bh.array(at), bh.array(b)).asnumpy(), a, b, dtype)
+
+
+@pytest.mark.gpu
+def test_gemm_infinities_stay_in_their_row_and_column():
+    import bohrium_amd as bh
+    for n in (20, 300, 1100):
+        a, b = np.ones((n, 37)), np.ones((37, n))
+        a[n // 2, 5] = np.inf
+        b[7, n - 1] = np.nan
+        c = bh.blas.gemm(bh.array(a), bh.array(b)).asnumpy()
+        assert np.isinf(c[n // 2, :-1]).all() and np.isnan(c[:, -1]).all()
+        c[n // 2] = 37
+        np.testing.assert_array_equal(c[:, :-1], np.full((n, n - 1), 37.0))
