@@ -910,6 +910,9 @@ std::vector<const bh_view *> Writer::preloadable(const LoopB &l) {
 // at a time.  A group is `unroll` consecutive elements on a one-rank walk without XCD parts (a
 // unit-stride view's loads merge into wide loads), else `unroll` elements strided by the grid.
 
+// Full reductions of at most this many elements can be one workgroup's (kernels of one code share it over their
+// sizes; from here on the autotuner works on the main loop).
+constexpr uint64_t kOneWorkgroupItems = 1u << 20;
 // Full reductions with at most this many instructions in their loop count as light (half the grid).
 constexpr size_t kLightReduceInstrs = 16;
 
@@ -2221,32 +2224,69 @@ void Writer::emit_full_reduce() {
         return "auto op_ = [](" + T + " x, " + T + " y) -> " + T + " { return " +
                combine_expr(a.instr->opcode, "x", "y") + "; };";
     };
+    // Store the results (in registers of thread 0) and run the tail.
+    auto results = [&](int ind) {
+        Scope fsc;
+        for (const Acc &a : accs) {
+            const bh_view &v = a.instr->operand[0];
+            if (a.is_tmp)
+                fsc.tmps.insert(v.base);
+            else
+                fsc.srep.insert(vkey(v));
+        }
+        std::set<std::string> stored;
+        for (const Acc &a : accs) {
+            if (a.is_tmp || !stored.insert(a.var).second) continue;
+            const bh_view &v = a.instr->operand[0];
+            indent(body, ind);
+            body << "a" << bid.at(v.base) << "[" << index(v) << "] = " << a.var << ";\n";
+        }
+        declare_scope(unit, fsc, ind);
+        for (size_t k = pos + 1; k < unit._block_list.size(); ++k) emit_block(unit._block_list[k], fsc, ind);
+        write_back(unit, fsc, ind);
+    };
+    // One workgroup has the whole result: it finishes the unit itself and the finalize launch (4 us of the 10 us
+    // that a sum of 1000 numbers takes on the device, and a launch on the host) is left out.  Not in the code of
+    // large reductions, whose main loop should not share registers with a tail.
+    // Only for a tail that shares no array with the loop: its thread would have to see the others' stores.
+    bool one = total <= kOneWorkgroupItems;
+    if (one) {
+        std::set<const bh_base *> outs, in_loop;
+        for (const Acc &a : accs) outs.insert(a.instr->operand[0].base);
+        for (const bh_base *b : l0.getAllBases())
+            if (!outs.count(b)) in_loop.insert(b);
+        for (size_t k = pos + 1; k < unit._block_list.size(); ++k)
+            for (const InstrPtr &i : jitk::allInstr(unit._block_list[k]))
+                for (const bh_view &v : i->operand)
+                    if (!bh_opcode_is_system(i->opcode) && !v.isConstant() && in_loop.count(v.base)) one = false;
+    }
     std::set<std::string> done;
     for (const Acc &a : accs) {
         if (!done.insert(a.var).second) continue;
         const std::string T = hip_type(a.t);
         body << "  { " << op_lambda(a) << "\n";
         body << "    " << a.var << " = bh_block_reduce(" << a.var << ", op_, (" << T << " *)bh_lds_);\n";
-        body << "    if (threadIdx.x == 0) *(" << T << " *)" << slot_addr(a, "bh_bid") << " = " << a.var << ";\n";
+        body << "    if (threadIdx.x == 0" << (one ? " && bh_nblk != 1" : "") << ") *(" << T << " *)" << slot_addr(a, "bh_bid")
+             << " = " << a.var << ";\n";
         body << "    __syncthreads(); }\n";
+    }
+    if (one) {
+        body << "  if (bh_nblk == 1 && threadIdx.x == 0) {\n";
+        results(2);
+        body << "  }\n";
+        kp.one_workgroup = true;
     }
     main_body = body.str();
     body.str("");
     body.clear();
 
     // Finalize kernel: fold the partials, store, run the tail in thread 0.
-    Scope fsc;
     done.clear();
+    if (one) body << "  if (bh_nparts == 1) return;\n";
     body << "  __shared__ __attribute__((aligned(16))) unsigned char bh_lds_[BH_WAVES * 16];\n";
     for (const Acc &a : accs) {
         if (!done.insert(a.var).second) continue;
         const std::string T = hip_type(a.t);
-        const bh_view &v = a.instr->operand[0];
-        if (a.is_tmp) {
-            fsc.tmps.insert(v.base);
-        } else {
-            fsc.srep.insert(vkey(v));
-        }
         body << "  " << T << " " << a.var << ";\n";
         body << "  { " << op_lambda(a) << "\n";
         body << "    " << T << " v_ = " << literal(jitk::sweep_identity(a.instr->opcode, a.t)) << ";\n";
@@ -2267,15 +2307,7 @@ void Writer::emit_full_reduce() {
         body << "    __syncthreads(); }\n";
     }
     body << "  if (threadIdx.x != 0) return;\n";
-    done.clear();
-    for (const Acc &a : accs) {
-        if (a.is_tmp || !done.insert(a.var).second) continue;
-        const bh_view &v = a.instr->operand[0];
-        body << "  a" << bid.at(v.base) << "[" << index(v) << "] = " << a.var << ";\n";
-    }
-    declare_scope(unit, fsc, 1);
-    for (size_t k = pos + 1; k < unit._block_list.size(); ++k) emit_block(unit._block_list[k], fsc, 1);
-    write_back(unit, fsc, 1);
+    results(1);
     kp.fin_name = "bh_kernel_fin";
 }
 

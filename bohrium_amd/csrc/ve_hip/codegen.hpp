@@ -66,6 +66,7 @@ struct KernelPlan {
      * workgroups right after `name` with the same arguments (folds the per-workgroup partials). */
     std::string fin_name;
     uint64_t fin_grid = 1;
+    bool one_workgroup = false;  // FULL_REDUCE: a grid of one workgroup needs no finalize launch
     std::vector<ArgSpec> args;
     /* The body as device functions (bh_main_, and bh_fin_ for FULL_REDUCE) and their parameters,
      * one per ArgSpec: declaration, value type and name.  `source` adds the kernels calling them. */

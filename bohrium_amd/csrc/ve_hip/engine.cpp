@@ -497,7 +497,7 @@ void EngineHip::launchPlan(KernelPlan &plan, const std::vector<bh_base *> &ord2b
         check(bhhip_compile(kPrelude, plan.source.c_str(), plan.name.c_str(), cache_dir.c_str(), nullptr),
               "kernel compilation");
         stats.time_compile += seconds_since(t);
-        if (!plan.fin_name.empty()) ++stats.launches;
+        if (!plan.fin_name.empty() && !(plan.one_workgroup && plan.grid == 1)) ++stats.launches;
         char hex[32];
         std::snprintf(hex, sizeof(hex), "%016llx", static_cast<unsigned long long>(plan.source_hash));
         dry_run_log.push_back(std::string(strategy_name(plan.strategy)) + " " + std::to_string(plan.grid) + " " +
@@ -532,7 +532,7 @@ void EngineHip::launchPlan(KernelPlan &plan, const std::vector<bh_base *> &ord2b
     ++stats.launches;
     errors_unchecked |= plan.uses_error_flag;
     if (recording != nullptr) recording->push_back({plan.function, plan.grid, plan.block, {buf, buf + n}});
-    if (plan.fin_function != nullptr) {
+    if (plan.fin_function != nullptr && !(plan.one_workgroup && plan.grid == 1)) {
         check(bhhip_launch(plan.fin_function, plan.fin_grid, plan.block, buf, n), "kernel launch");
         ++stats.launches;
         if (recording != nullptr) recording->push_back({plan.fin_function, plan.fin_grid, plan.block, {buf, buf + n}});
