@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <map>
 #include <set>
+#include <unordered_set>
 
 #include <bohrium/bh_opcode.h>
 
@@ -242,19 +243,29 @@ constexpr int64_t kRecomputeBytes = 1 << 20;
 } // namespace
 
 int recompute_temporaries(std::vector<bh_instruction *> &list, RewriteStore &store, const std::set<bh_base *> &syncs) {
-    bool sweeps = false;
+    // Only what an instruction behind a reduction reads can be worth repeating (this runs on every flush: one
+    // pass over the list, and the others only for the few candidates).
+    std::unordered_set<const bh_base *> read_late;
+    bool reduced_before = false;
     for (const bh_instruction *i : list) {
         if (i->opcode > BH_MAX_OPCODE_ID) return 0;
-        sweeps |= bh_opcode_is_reduction(i->opcode) != 0;
+        if (reduced_before && i->opcode != BH_FREE)
+            for (size_t o = 1; o < i->operand.size(); ++o) {
+                const bh_view &v = i->operand[o];
+                if (!v.isConstant() && v.base->nbytes() >= kRecomputeBytes) read_late.insert(v.base);
+            }
+        reduced_before |= bh_opcode_is_reduction(i->opcode) != 0;
     }
-    if (!sweeps) return 0;
+    if (read_late.empty()) return 0;
     int count = 0;
     for (size_t k = 0; k < list.size(); ++k) {
         const bh_instruction *p = list[k];
-        if (!cheap(p->opcode) || p->operand.size() < 2 || !full_contiguous(p->operand[0])) continue;
+        if (!cheap(p->opcode) || p->operand.size() < 2 || !read_late.count(p->operand[0].base) ||
+            !full_contiguous(p->operand[0]))
+            continue;
         const bh_view out = p->operand[0];
         bh_base *T = out.base;
-        if (T->nbytes() < kRecomputeBytes || syncs.count(T)) continue;
+        if (syncs.count(T)) continue;
         // Written here only, freed in this flush, read through its whole view only.
         bool ok = true;
         size_t freed = kNone;
