@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <map>
 #include <set>
+#include <unordered_map>
 #include <unordered_set>
 
 #include <bohrium/bh_opcode.h>
@@ -239,21 +240,29 @@ int64_t distinct_elements(const bh_view &v) {
 
 // Smaller results stay in the caches between the kernels that share them.
 constexpr int64_t kRecomputeBytes = 1 << 20;
+constexpr size_t kRecomputeList = 4096;
 
 } // namespace
 
 int recompute_temporaries(std::vector<bh_instruction *> &list, RewriteStore &store, const std::set<bh_base *> &syncs) {
-    // Only what an instruction behind a reduction reads can be worth repeating (this runs on every flush: one
-    // pass over the list, and the others only for the few candidates).
+    // This runs on every flush: one pass over the list finds what is read twice and behind a reduction, and the
+    // others are only for those few.  A list far beyond the front end's flush threshold of 1000 instructions is left
+    // alone, since each candidate costs passes over it.
+    if (list.size() > kRecomputeList) return 0;
+    std::unordered_map<const bh_base *, int> reads;
     std::unordered_set<const bh_base *> read_late;
     bool reduced_before = false;
     for (const bh_instruction *i : list) {
         if (i->opcode > BH_MAX_OPCODE_ID) return 0;
-        if (reduced_before && i->opcode != BH_FREE)
+        if (i->opcode != BH_FREE) {
+            const bh_base *last = nullptr;  // (c * c reads c once)
             for (size_t o = 1; o < i->operand.size(); ++o) {
                 const bh_view &v = i->operand[o];
-                if (!v.isConstant() && v.base->nbytes() >= kRecomputeBytes) read_late.insert(v.base);
+                if (v.isConstant() || v.base == last || v.base->nbytes() < kRecomputeBytes) continue;
+                last = v.base;
+                if (++reads[v.base] > 1 && reduced_before) read_late.insert(v.base);
             }
+        }
         reduced_before |= bh_opcode_is_reduction(i->opcode) != 0;
     }
     if (read_late.empty()) return 0;

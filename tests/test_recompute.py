@@ -81,3 +81,26 @@ def test_results_do_not_change(dtype):
         np.testing.assert_array_equal(g, p)
         # sums of up to 2^20 terms of size at most 64, order free: sqrt(terms) eps with a factor of 8
         np.testing.assert_allclose(g, w, rtol=8 * 1024 * eps, atol=8 * 1024 * eps * np.abs(w).max())
+
+
+def test_a_long_list_is_left_alone():
+    """A flush far beyond the flush threshold (thousands of small arrays) is not searched: 1200 arrays of their own sizes
+    in front of a program that is rewritten by itself, and 300, which still are a list that is."""
+    prog = r"""
+import sys
+sys.path.insert(0, %r)
+exec(%r)
+from bohrium_amd import _bh_api
+_bh_api.set_flush_threshold(10 ** 7)
+x = bh.empty((2048, 512), np.float32)
+ys = [bh.empty((256 + k,), np.float32) for k in range(1200)]
+bh.flush()
+for count in (1200, 300):
+    keep = [((y * 2.0 + 1.0).sum()) for y in ys[:count]] + both(x, 1)
+    bh.flush()
+    print([l for l in bh.message("statistic").splitlines() if l.startswith("recomputed")][0].split()[1])
+""" % (ROOT, PROGRAMS)
+    r = subprocess.run([sys.executable, "-c", prog], env=dict(os.environ, BH_HIP_DRY_RUN="1"), text=True,
+                       stdout=subprocess.PIPE, stderr=subprocess.STDOUT, timeout=600)
+    assert r.returncode == 0, r.stdout[-3000:]
+    assert r.stdout.split() == ["0", "1"], r.stdout
