@@ -338,7 +338,7 @@ public:
      * most their own workgroup count): fewer, longer tasks than their standalone grid.  0: the plan's
      * own grid. */
     int persist_items = 16384;
-    int persist_grid = 0;  // >0: at most this many workgroups in the persistent launch
+    int persist_grid = 0;  // at most this many workgroups in the persistent launch (0: one per CU)
     /* Polls of a grid barrier's wait before it gives up and raises the error flag (default 2^22,
      * seconds of waiting; a tiny value forces the error path from the host). */
     unsigned persist_spin = 1u << 22;
