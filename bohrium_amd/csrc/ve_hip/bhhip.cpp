@@ -260,7 +260,7 @@ int bhhip_launch(void *function, uint64_t grid, uint32_t block, const void *args
     void *config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, const_cast<void *>(args), HIP_LAUNCH_PARAM_BUFFER_SIZE, &size,
                       HIP_LAUNCH_PARAM_END};
     if (grid == 0) return 0;
-    if (grid > 0x7fffffffull) {
+    if (grid > 0x7fffffffull || grid * block > 0xffffffffull) {  // workgroups, threads
         g_err = "bhhip_launch: grid too large";
         return 1;
     }

@@ -1407,11 +1407,48 @@ struct SegForm {
     std::vector<InstrPtr> post;
     std::set<const bh_base *> loop_temps;  // temporaries of P that only C uses
     bool columns = false;  // the contiguous axis is P's (reduce over rows), else C's
-    int width = 1;         // elements of the contiguous axis that 16 bytes of the widest such view hold
+    /* The launch: V neighbours of the contiguous axis per thread and load (16 bytes of the widest view along it),
+     * U loads in flight; columns: w threads along the outputs, else `lanes` threads per output; row_blocks
+     * workgroups cover the outputs, times `splits` pieces of `chunk` elements of the reduced axis. */
+    int V = 1, U = 4;
+    uint64_t outs_n = 1, lanes = 1, row_blocks = 1, splits = 1, chunk = 1, w = 1;
 };
 
 // Shapes below this many elements keep the row and map skeletons (one small launch, batchable).
 constexpr uint64_t kSegMinItems = 1u << 16;
+
+// The reduced axis is cut until the launch has about this many workgroups.
+constexpr uint64_t kSegBlocks = 2048;
+
+void seg_launch(SegForm &f, int width, int64_t inner, uint64_t W) {
+    const uint64_t R = static_cast<uint64_t>(f.C->size);
+    f.V = width;
+    f.U = f.columns ? (f.V >= 4 ? 4 : 8) : 4;
+    f.chunk = R;
+    const uint64_t U = static_cast<uint64_t>(f.U);
+    if (f.columns) {
+        while (inner % f.V != 0) f.V /= 2;  // a thread's outputs are V neighbours of one innermost row
+        const uint64_t groups = f.outs_n / static_cast<uint64_t>(f.V);
+        f.row_blocks = (groups + W - 1) / W;
+        f.w = (groups + f.row_blocks - 1) / f.row_blocks;
+        const uint64_t step = W / f.w * U;
+        f.splits = std::max<uint64_t>(1, std::min((kSegBlocks + f.row_blocks - 1) / f.row_blocks, R / (2 * step)));
+        f.chunk = (R + f.splits - 1) / f.splits;
+    } else {
+        // A workgroup per row for long rows (and for moderate ones when there are few), else a wave, and
+        // fewer lanes for short rows: each lane loads at least twice.
+        const uint64_t V = static_cast<uint64_t>(f.V), wide = W * 2 * V;
+        f.lanes = R >= wide * U || (f.outs_n < kSegBlocks && R >= wide) ? W : 64;
+        while (f.lanes > 4 && f.lanes <= 64 && f.lanes * 2 * V > R) f.lanes /= 2;
+        const uint64_t per_block = W / f.lanes;
+        f.row_blocks = (f.outs_n + per_block - 1) / per_block;
+        if (f.lanes == W)
+            f.splits = std::max<uint64_t>(1, std::min((kSegBlocks + f.row_blocks - 1) / f.row_blocks, R / (2 * f.lanes * V * U)));
+        f.chunk = (R + f.splits - 1) / f.splits;
+        f.chunk = (f.chunk + f.lanes * V - 1) / (f.lanes * V) * (f.lanes * V);
+    }
+    f.splits = (R + f.chunk - 1) / f.chunk;
+}
 
 SegForm seg_form(const LoopB &l0, const std::set<const bh_base *> &params) {
     SegForm none, f;
@@ -1524,7 +1561,11 @@ SegForm seg_form(const LoopB &l0, const std::set<const bh_base *> &params) {
         }
     if (rows == cols) return none;
     f.columns = cols > rows;
-    f.width = std::max(1, std::min(4, 16 / widest));
+    f.outs_n = outs_n;
+    const uint64_t W = KernelPlan().block;
+    seg_launch(f, std::max(1, std::min(4, 16 / widest)), P.size, W);
+    // (a launch holds fewer than 2^32 threads, and this skeleton has a thread group for every output)
+    if (f.row_blocks * f.splits * W >= 1ull << 32) return none;
     return f;
 }
 
@@ -1535,8 +1576,6 @@ SegForm seg_form(const LoopB &l0, const std::set<const bh_base *> &params) {
 // axis is cut into `splits` pieces until the launch has about kSegBlocks workgroups.  Measured on float32:
 // mean, variance and standardised matrix of 100000 x 500 by columns 1792 -> 231 us (the two reduction
 // kernels 0.81 and 0.88 ms before), of 16384 x 3000 by rows 223 -> 198 us (4-byte loads before).
-constexpr uint64_t kSegBlocks = 2048;
-
 void Writer::emit_seg_reduce() {
     const LoopB &l0 = unit._block_list.back().getLoop();
     const uint64_t p = std::max<uint64_t>(1, jitk::parallel_ranks(l0).first);
@@ -1544,48 +1583,17 @@ void Writer::emit_seg_reduce() {
     const SegForm f = seg_form(l0, std::set<const bh_base *>(kp.params.begin(), kp.params.end()));
     if (f.C == nullptr) throw std::logic_error("seg skeleton: block has another form");
     for (const bh_instruction *i : f.seeds) skip.insert(i);
-    const LoopB &C = *f.C, &P = *chain[p - 1];
-    uint64_t outs_n = 1;
-    for (uint64_t r = 0; r < p; ++r) outs_n *= static_cast<uint64_t>(chain[r]->size);
-    const uint64_t R = static_cast<uint64_t>(C.size);
-    kp.work_items = outs_n * R;
-    const uint64_t W = kp.block;
+    const LoopB &C = *f.C;
+    const uint64_t outs_n = f.outs_n, W = kp.block;
+    kp.work_items = outs_n * static_cast<uint64_t>(C.size);
     const std::string rk = std::to_string(C.rank), pk = std::to_string(p - 1);
     const std::string nR = "n" + std::to_string(lid.at(&C));
-
-    // Vector width, threads along the outputs / lanes per row, splits of the reduced axis.
-    int V = f.width;
-    const int U = f.columns ? (V >= 4 ? 4 : 8) : 4;
-    uint64_t lanes = 1, row_blocks = 1, splits = 1, chunk = R, w = 1;
-    if (f.columns) {
-        while (P.size % V != 0) V /= 2;  // a thread's outputs are V neighbours of one innermost row
-        const uint64_t groups = outs_n / static_cast<uint64_t>(V);
-        row_blocks = (groups + W - 1) / W;
-        w = (groups + row_blocks - 1) / row_blocks;
-        const uint64_t ty = W / w;
-        const uint64_t step = ty * static_cast<uint64_t>(U);
-        splits = std::max<uint64_t>(1, std::min((kSegBlocks + row_blocks - 1) / row_blocks, R / (2 * step)));
-        chunk = (R + splits - 1) / splits;
-        splits = (R + chunk - 1) / chunk;
-    } else {
-        // A workgroup per row for long rows (and for moderate ones when there are few), else a wave, and
-        // fewer lanes for short rows: each lane loads at least twice.
-        const uint64_t wide = W * static_cast<uint64_t>(2 * V);
-        lanes = R >= wide * static_cast<uint64_t>(U) || (outs_n < kSegBlocks && R >= wide) ? W : 64;
-        while (lanes > 4 && lanes <= 64 && lanes * static_cast<uint64_t>(2 * V) > R) lanes /= 2;
-        const uint64_t per_block = W / lanes;
-        row_blocks = (outs_n + per_block - 1) / per_block;
-        const uint64_t step = lanes * static_cast<uint64_t>(V * U);
-        if (lanes == 256)
-            splits = std::max<uint64_t>(1, std::min((kSegBlocks + row_blocks - 1) / row_blocks, R / (2 * step)));
-        chunk = (R + splits - 1) / splits;
-        chunk = (chunk + lanes * V - 1) / (lanes * V) * (lanes * V);
-        splits = (R + chunk - 1) / chunk;
-    }
+    const int V = f.V, U = f.U;
+    const uint64_t lanes = f.lanes, row_blocks = f.row_blocks, splits = f.splits;
     const bool split = splits > 1;
     kp.grid = row_blocks * splits;
-    shape_args = {{"sg_nb", static_cast<int64_t>(row_blocks)}, {"sg_ch", static_cast<int64_t>(chunk)}};
-    if (f.columns) shape_args.emplace_back("sg_w", static_cast<int64_t>(w));
+    shape_args = {{"sg_nb", static_cast<int64_t>(row_blocks)}, {"sg_ch", static_cast<int64_t>(f.chunk)}};
+    if (f.columns) shape_args.emplace_back("sg_w", static_cast<int64_t>(f.w));
 
     struct Acc {
         InstrPtr instr;
