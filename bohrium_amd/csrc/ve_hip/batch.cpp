@@ -43,6 +43,10 @@ void check(int rc, const char *what) {
 
 uint64_t round_up(uint64_t n, uint64_t m) { return (n + m - 1) / m * m; }
 
+// LDS tiles of all codes in one persistent kernel (its LDS is their sum): half of a CU's 160 KB, so that two
+// workgroups still share a CU.
+constexpr uint64_t kPersistTileBytes = 80 << 10;
+
 /* The workgroup table of a batched launch (batch_source) from the items' workgroup counts; sets the
  * launch's `items` argument and its total workgroups.  Grid-stride and reduction skeletons: the first
  * workgroup of each item and the end.
@@ -140,8 +144,9 @@ std::unique_ptr<EngineHip::PersistPlan> EngineHip::buildPersist(CachedFlush &cf)
     std::unique_ptr<PersistPlan> pp(new PersistPlan());
     std::unordered_map<uint64_t, uint32_t> code_of;
     std::vector<uint32_t> plan_code;
+    uint64_t tile_bytes = 0;
     // Every plan must fit the persistent kernel: 256-thread workgroups, a skeleton whose body only
-    // uses its workgroup number and count (or a ticket), and few distinct codes.
+    // uses its workgroup number and count (or a ticket), few distinct codes, and tiles that fit the LDS together.
     auto add = [&](const PlanRef &r) -> bool {
         const KernelPlan &p = cf.kernels[r.kernel].plans[r.plan];
         if (p.block != 256 || p.grid == 0 || p.grid > 0x7fffffffull) return false;
@@ -150,7 +155,8 @@ std::unique_ptr<EngineHip::PersistPlan> EngineHip::buildPersist(CachedFlush &cf)
             return false;
         auto it = code_of.find(p.source_hash);
         if (it == code_of.end()) {
-            if (pp->codes.size() >= 32) return false;
+            tile_bytes += p.tile_bytes;
+            if (pp->codes.size() >= 32 || tile_bytes > kPersistTileBytes) return false;
             it = code_of.emplace(p.source_hash, static_cast<uint32_t>(pp->codes.size())).first;
             pp->codes.push_back(&p);
         }
@@ -231,10 +237,15 @@ std::unique_ptr<EngineHip::PersistPlan> EngineHip::buildPersist(CachedFlush &cf)
 bool EngineHip::launchPersist(PersistPlan &pp, CachedFlush &cf, const std::vector<bh_base *> &ord2base,
                               const std::vector<bh_instruction *> &instrs) {
     auto t = std::chrono::steady_clock::now();
+    if (pp.refused) return false;
     if (pp.fn == nullptr) {
         const std::string src = persist_source(pp.codes);
-        check(bhhip_compile(kPreludeRef(), src.c_str(), "bh_kernel_persist", cache_dir.c_str(), &pp.fn),
-              "kernel compilation");
+        if (bhhip_compile(kPreludeRef(), src.c_str(), "bh_kernel_persist", cache_dir.c_str(), &pp.fn) != 0) {
+            // (each code compiles by itself: their sum has met a limit) the levels run instead
+            pp.refused = true;
+            ++persist_fallbacks;
+            return false;
+        }
         // Every workgroup must be resident at once (the grid barriers wait for all of them); a
         // multiple of 8 keeps a task's XCD that of its position in its level.
         int per_cu = 0, cus = 0;

@@ -1876,8 +1876,10 @@ void Writer::emit_map_tiled(const TiledForm &f, const std::vector<const LoopB *>
     uint64_t tiles = static_cast<uint64_t>((chain[a]->size + T - 1) / T) * static_cast<uint64_t>((chain[f.q]->size + T - 1) / T);
     for (int64_t r = 0; r < a; ++r)
         if (r != f.q) tiles *= static_cast<uint64_t>(chain[r]->size);
-    for (size_t k = 0; k < f.views.size(); ++k)
+    for (size_t k = 0; k < f.views.size(); ++k) {
+        kp.tile_bytes += static_cast<uint64_t>(T * (T + 1) * bh_type_size(f.views[k]->base->dtype()));
         body << "  __shared__ " << hip_type(f.views[k]->base->dtype()) << " tl" << k << "_[" << T * (T + 1) << "];\n";
+    }
     const std::string sT = std::to_string(T), qi = "i" + std::to_string(f.q), ai = "i" + std::to_string(a);
     body << "  const int64_t ta_ = (" << n(a) << " + " << T - 1 << ") / " << T << ", tb_ = (" << n(f.q) << " + " << T - 1
          << ") / " << T << ";\n  int64_t tiles_ = ta_ * tb_;\n";

@@ -67,6 +67,7 @@ struct KernelPlan {
     std::string fin_name;
     uint64_t fin_grid = 1;
     bool one_workgroup = false;  // FULL_REDUCE: a grid of one workgroup needs no finalize launch
+    uint64_t tile_bytes = 0;     // MAP: LDS tiles of transposed operands (the other skeletons hold a few hundred bytes)
     std::vector<ArgSpec> args;
     /* The body as device functions (bh_main_, and bh_fin_ for FULL_REDUCE) and their parameters,
      * one per ArgSpec: declaration, value type and name.  `source` adds the kernels calling them. */

@@ -296,6 +296,7 @@ private:
         uint32_t max_level_tasks = 0;
         void *fn = nullptr;
         uint32_t grid = 0;
+        bool refused = false;  // the codes do not compile as one kernel: the levels run
         unsigned char *dev = nullptr;  // tasks | levels | barrier counters (16 bytes) | arguments
         uint64_t dev_bytes = 0, args_at = 0;
         bool tables_uploaded = false;
