@@ -353,13 +353,29 @@ void indent(std::ostringstream &o, int n) { o << std::string(n * 2, ' '); }
 
 // ------------------------------------------------------------------ writer
 
-// Arrays from this size on are stored past the caches (non-temporal): such a result and its input exceed the 256 MB
-// last-level cache anyway, and what is kept out of it stays for the input's next reader.  Measured: x*2+1 of 2^28
-// float32 392 -> 379 us, 200 sweeps of the 8192^2 stencil 23.9 -> 22.1 ms, and where three kernels read one 197 MB
-// array before the result is stored, row statistics 156 -> 126 us and column statistics 176 -> 147 us.  The stores
-// of a wave have to be contiguous: a scan with 32 bytes between its lanes' 16-byte stores went from 217 to 376 us,
-// with contiguous ones 206 us.
-constexpr int64_t kStreamBytes = 128ll << 20;
+// Results are stored past the caches (non-temporal) when the kernel's arrays exceed the 256 MB last-level cache by a
+// quarter: they would not stay there anyway, and what is kept out of it stays for the input's next reader.  Measured:
+// 200 sweeps of the 8192^2 float32 stencil 23.9 -> 22.1 ms; where three kernels read one 197 MB array before the
+// result is stored, row statistics 156 -> 126 us and column statistics 176 -> 147 us; x*2+1 and two maps that read the
+// result, 256 MiB arrays 330 -> 305 us, 160 MiB arrays (the limit) 208 -> 188, but 130 MiB arrays 145 -> 157.
+// Only where they pay, which the same measurements bound:
+//  - the lanes store neighbouring pieces of at most 16 bytes.  y[::8] = s*2 into 1 GiB 516 -> 1666 us with
+//    non-temporal stores, g.T[...] = q*2 4.5 -> 12.3 ms, 1 GiB of bool -> int64 354 -> 712 us at 32 bytes a lane, but
+//    238 -> 190 at 16;
+//  - rows of the written view, where it is not contiguous, that hold a wave's store (64 lanes of 16 bytes);
+//  - the kernel reads at least an eighth of what it stores.  400 MiB written and nothing read: 72 -> 96 us.
+constexpr int64_t kStreamBytes = 320ll << 20;
+constexpr int64_t kStreamStore = 128ll << 20;  // (a smaller result beside large inputs stays for its reader)
+constexpr int64_t kStreamRead = 8;
+constexpr int64_t kStreamRow = 64 * 16;
+
+// Bytes of the base that a view reaches (broadcast axes count once).
+int64_t reached_bytes(const bh_view &v) {
+    int64_t n = bh_type_size(v.base->dtype());
+    for (int64_t d = 0; d < v.ndim; ++d)
+        if (v.stride[d] != 0) n *= v.shape[d];
+    return n;
+}
 
 struct KernelParam {
     std::string type;  // value type: "double *", "int64_t", ...
@@ -531,10 +547,12 @@ private:
     }
     std::string const_ref(const bh_instruction &i) { return "c" + std::to_string(const_of_origin.at(i.origin_id)); }
 
-    /* Arrays at least as large as the last-level cache are stored past it. */
-    static bool streamed(const bh_base *b) {
-        return b->nbytes() >= kStreamBytes && !bh_type_is_complex(b->dtype());
-    }
+    /* The rank that the lanes of a wave walk in the code being written (-1: one thread, or no such rank), and the
+     * neighbouring elements of it that one lane owns. */
+    int64_t lane_axis = -1;
+    int lane_run = 1;
+    /* Whether stores to `v` go past the caches (kStreamBytes). */
+    bool streamed(const bh_view &v) const;
     void declare_scope(const LoopB &l, Scope &sc, int ind);
     void write_back(const LoopB &l, Scope &sc, int ind);
     void emit_block(const Block &b, Scope &sc, int ind);
@@ -661,6 +679,30 @@ void Writer::collect() {
             if (v.hasSlide()) sliding_src[&v] = {i->origin_id, static_cast<int>(o)};
         }
     }
+}
+
+bool Writer::streamed(const bh_view &v) const {
+    if (lane_axis < 0 || v.ndim <= lane_axis || v.stride[lane_axis] != 1 || bh_type_is_complex(v.base->dtype())) return false;
+    const int64_t size = bh_type_size(v.base->dtype());
+    if (lane_run * size > 16) return false;
+    if (!v.isContiguous() && v.shape[lane_axis] * size < kStreamRow) return false;
+    // The kernel's arrays, by what it reaches of each.
+    std::map<const bh_base *, int64_t> all, read;
+    for (const InstrPtr &i : jitk::allInstr(unit)) {
+        if (bh_opcode_is_system(i->opcode)) continue;
+        for (size_t o = 0; o < i->operand.size(); ++o) {
+            const bh_view &w = i->operand[o];
+            if (w.isConstant() || std::find(kp.params.begin(), kp.params.end(), w.base) == kp.params.end()) continue;
+            const int64_t n = reached_bytes(w);
+            all[w.base] = std::max(all[w.base], n);
+            if (o > 0) read[w.base] = std::max(read[w.base], n);
+        }
+    }
+    int64_t total = 0, loaded = 0;
+    for (const auto &b : all) total += b.second;
+    for (const auto &b : read) loaded += b.second;
+    const int64_t stored = reached_bytes(v);
+    return total >= kStreamBytes && stored >= kStreamStore && loaded * kStreamRead >= stored;
 }
 
 void Writer::declare_scope(const LoopB &l, Scope &sc, int ind) {
@@ -810,7 +852,7 @@ void Writer::emit_instr(const bh_instruction &instr, Scope &sc, int ind) {
         }
     }
     const bh_view &out = instr.operand[0];
-    if (sc.isArray(out) && !bh_opcode_is_sweep(instr.opcode) && instr.opcode != BH_COND_SCATTER && streamed(out.base)) {
+    if (sc.isArray(out) && !bh_opcode_is_sweep(instr.opcode) && instr.opcode != BH_COND_SCATTER && streamed(out)) {
         const std::string at = ops[0];
         ops[0] = "nt_";
         body << "{ " << hip_type(out.base->dtype()) << " nt_; " << hip_operation(instr, ops, cfg.math64)
@@ -1010,6 +1052,8 @@ bool Writer::stencil_walk(const Element &e, const std::string &n0, const std::st
     int64_t H = 8 * UR;
     while (H > UR && ((s0 + H - 1) / H) * groups < 256ll * 8 * kp.block) H -= UR;
     shape_args.emplace_back("st_h", H);
+    lane_axis = 1;
+    lane_run = V;
     *tasks = (s0 + H - 1) / H * groups;
 
     // Columns of window k that row j of a row group needs: those of the taps that touch it.
@@ -1147,7 +1191,8 @@ void Writer::grid_stride(const std::string &tot_in, int unroll, const Element &e
         body << "  const int64_t st_ = (int64_t)bh_nblk * BH_WG;\n";
         body << "  int64_t g_ = (int64_t)bh_bid * BH_WG + threadIdx.x;\n";
     }
-    if (unroll > 1 && e.unit && !parts) {
+    lane_run = unroll > 1 && e.unit && !parts ? unroll : 1;
+    if (lane_run > 1) {
         // Groups of `unroll` consecutive elements: group q_ is [q_ * unroll, q_ * unroll + unroll), the
         // groups are walked grid-stride, so a lane's loads of one unit-stride view are adjacent (the
         // compiler merges them into one wide load, e.g. 16 bytes for 4 floats) and a wave's lanes read
@@ -1379,6 +1424,7 @@ void Writer::emit_row_reduce() {
     }
     Scope &ps = scopes[p - 1];
     const int ind = 2 + static_cast<int>(p);
+    lane_axis = chain[p - 1]->rank + 1;
     // The row's own instructions run in every lane (same values); each lane loop is strided by the
     // lanes and its reductions are folded across the wave right after it (emit_block).
     emit_blocks(*chain[p - 1], ps, ind);
@@ -1592,6 +1638,8 @@ void Writer::emit_seg_reduce() {
     const uint64_t lanes = f.lanes, row_blocks = f.row_blocks, splits = f.splits;
     const bool split = splits > 1;
     kp.grid = row_blocks * splits;
+    lane_axis = f.columns ? static_cast<int64_t>(p) - 1 : C.rank;
+    lane_run = V;
     shape_args = {{"sg_nb", static_cast<int64_t>(row_blocks)}, {"sg_ch", static_cast<int64_t>(f.chunk)}};
     if (f.columns) shape_args.emplace_back("sg_w", static_cast<int64_t>(f.w));
 
@@ -1872,6 +1920,7 @@ void Writer::emit_seg_reduce() {
 void Writer::emit_map_tiled(const TiledForm &f, const std::vector<const LoopB *> &chain, uint64_t p, const Scope &ksc) {
     const int64_t a = static_cast<int64_t>(p) - 1;
     const int T = f.side, per = T * T / 256, rows = 256 / T;
+    lane_axis = a;
     auto n = [&](int64_t r) { return "n" + std::to_string(lid.at(chain[r])); };
     uint64_t tiles = static_cast<uint64_t>((chain[a]->size + T - 1) / T) * static_cast<uint64_t>((chain[f.q]->size + T - 1) / T);
     for (int64_t r = 0; r < a; ++r)
@@ -1972,6 +2021,7 @@ void Writer::emit_map() {
     for (uint64_t r = 0; r < p; ++r) body << " * n" << lid.at(chain[r]);
     body << ";\n";
     // Only loops without inner sequential work are unrolled (their body is straight-line code).
+    lane_axis = static_cast<int64_t>(p) - 1;
     const bool flat = p == 1 ? l0.isInnermost() : chain[p - 1]->isInnermost();
     if (flat && p > 1) {
         const TiledForm f = tiled_form(chain, p, preloadable(*chain[p - 1]));
@@ -2175,6 +2225,7 @@ void Writer::emit_full_reduce() {
                std::to_string(slot.at(a.var)) + ") * 16)";
     };
     declare_scope(unit, ksc, 1);
+    lane_axis = pairs.empty() ? 0 : 1;
     if (!pairs.empty()) {
         // One flat grid-stride loop over (i0, i1); each row temporary is the accumulator
         // of the rank-0 reduction it feeds.
@@ -2234,6 +2285,7 @@ void Writer::emit_full_reduce() {
         return "auto op_ = [](" + T + " x, " + T + " y) -> " + T + " { return " +
                combine_expr(a.instr->opcode, "x", "y") + "; };";
     };
+    lane_axis = -1;
     // Store the results (in registers of thread 0) and run the tail.
     auto results = [&](int ind) {
         Scope fsc;
@@ -2352,6 +2404,8 @@ void Writer::emit_scan() {
         while (items % V != 0) V /= 2;
     }
     const int groups = items / V;
+    lane_axis = 0;
+    lane_run = V;
     const int64_t ntiles = (l0.size + tile_elems - 1) / tile_elems;
     kp.grid = static_cast<uint64_t>(std::max<int64_t>(1, ntiles));
     // Scratch layout: [tile counter u64 = epoch << 32 | tiles taken, pad to 256], then one record
@@ -2464,7 +2518,7 @@ void Writer::emit_scan() {
         const std::string at = "a" + std::to_string(bid.at(out.base)) + "[" + index(out) + "]";
         const std::string value = "op_(p_, v_[j_ * " + std::to_string(V) + " + e_])";
         body << (full ? "    " : "    if (i0 < n" + std::to_string(lid.at(&l0)) + ") ")
-             << (streamed(out.base) ? "__builtin_nontemporal_store(" + value + ", &" + at + ")" : at + " = " + value)
+             << (streamed(out) ? "__builtin_nontemporal_store(" + value + ", &" + at + ")" : at + " = " + value)
              << ";\n  }\n  }\n";
     }
     body << "  }\n";
