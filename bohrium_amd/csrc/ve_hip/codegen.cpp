@@ -353,18 +353,20 @@ void indent(std::ostringstream &o, int n) { o << std::string(n * 2, ' '); }
 
 // ------------------------------------------------------------------ writer
 
-// Results are stored past the caches (non-temporal) when the kernel's arrays exceed the 256 MB last-level cache by a
-// quarter: they would not stay there anyway, and what is kept out of it stays for the input's next reader.  Measured:
-// 200 sweeps of the 8192^2 float32 stencil 23.9 -> 22.1 ms; where three kernels read one 197 MB array before the
-// result is stored, row statistics 156 -> 126 us and column statistics 176 -> 147 us; x*2+1 and two maps that read the
-// result, 256 MiB arrays 330 -> 305 us, 160 MiB arrays (the limit) 208 -> 188, but 130 MiB arrays 145 -> 157.
+// Results are stored past the caches (non-temporal) when the kernel's arrays together fill the 256 MB last-level cache:
+// they would not stay there anyway, and what is kept out of it stays for the input's next reader.  Measured, cached ->
+// non-temporal: 200 sweeps of the 8192^2 float32 stencil 23.9 -> 22.1 ms; where three kernels read one 197 MB array before
+// the result is stored, row statistics 156 -> 126 us and column statistics 176 -> 147 us; x*2+1 into 256 MiB 105 -> 83 us,
+// into 144 MiB 52 -> 45, into 128 (256 with its input) 42.8 -> 40.3, and with the result's maximum taken next 68 -> 67;
+// running counts of 22e6 float32 (255 MiB) 96 -> 85.  Below the limit the two are level: of 17e6 (195 MiB) 78 and 81, int16 -> float32
+// into 152 MiB 38.2 and 37.9.
 // Only where they pay, which the same measurements bound:
 //  - the lanes store neighbouring pieces of at most 16 bytes.  y[::8] = s*2 into 1 GiB 516 -> 1666 us with
 //    non-temporal stores, g.T[...] = q*2 4.5 -> 12.3 ms, 1 GiB of bool -> int64 354 -> 712 us at 32 bytes a lane, but
 //    238 -> 190 at 16;
 //  - rows of the written view, where it is not contiguous, that hold a wave's store (64 lanes of 16 bytes);
 //  - the kernel reads at least an eighth of what it stores.  400 MiB written and nothing read: 72 -> 96 us.
-constexpr int64_t kStreamBytes = 320ll << 20;
+constexpr int64_t kStreamBytes = 240ll << 20;
 constexpr int64_t kStreamStore = 128ll << 20;  // (a smaller result beside large inputs stays for its reader)
 constexpr int64_t kStreamRead = 8;
 constexpr int64_t kStreamRow = 64 * 16;

@@ -16,9 +16,11 @@ M = 1 << 20
 # name: (program over the large arrays, whether it stores past the caches)
 PROGRAMS = {
     "flat": ("f * 2 + 1", True),
-    "below the limit": ("f[:39 * M] * 2", False),
-    "at the limit": ("f[:40 * M] * 2", True),
-    "in place, 256 MiB": ("f.__imul__(2)", False),
+    "a small result": ("f[:31 * M] * 2", False),
+    "large enough": ("f[:32 * M] * 2", True),
+    "below the limit": ("b[:47 * M].astype(np.float32)", False),
+    "above the limit": ("b[:49 * M].astype(np.float32)", True),
+    "in place, 192 MiB": ("f[:48 * M].__imul__(2)", False),
     "double, 16 bytes a lane": ("unrolled(2, lambda: d * 2)", True),
     "double, 32 bytes a lane": ("unrolled(4, lambda: d * 2)", False),
     "strided": ("put(f[::8], f[:8 * M] * 2)", False),
