@@ -1462,8 +1462,28 @@ struct SegForm {
     uint64_t outs_n = 1, lanes = 1, row_blocks = 1, splits = 1, chunk = 1, w = 1;
 };
 
-// Shapes below this many elements keep the row and map skeletons (one small launch, batchable).
+// Where one reduction is segmented, from device times of sums of x * x in float32 and float64 (one launch and its gap
+// are 6 us of them; a second one, the finalize, adds 2.3 us and 3 us on the host).
+// Rows, lanes along the row: from 2^16 elements on the skeletons are level (256^2: 6.1 us) or this one is ahead (8 x
+// 8192: row 16.6, seg 6.1 us; 131072 x 16: map 8.0, seg 6.3).
+// Columns are split and finalized, so the row skeleton's single launch wins while its waves' walks down the columns
+// are short and their lines stay in the L2s: row / seg 2048 x 256 8.6 / 9.4 us, 512 x 2048 6.7 / 9.4, 1024 x 1500 11.1 / 8.8
+// (host and device together 11.5 / 14.6); 4096 x 16 11.7 / 8.2, 2048 x 700 16.1 / 9.0, 40 x 60000 15.8 / 9.7.
+// Fewer than 32 rows: a thread per column reads them coalesced in one launch.  map / seg 16 x 2^20 float32 14.7 / 40.3, 31 x 2^18
+// 8.3 / 17.4; 16-byte loads without a split are ahead: 16 x 2^22 64 / 51, 31 x 2^21 56 / 47.
+// With a map over the outputs in its finalize (a mean) this skeleton has no launch more: x - x.mean(0) of 256^2 18.5 / 15.3
+// us, of 1024^2 22.1 / 15.5.
 constexpr uint64_t kSegMinItems = 1u << 16;
+constexpr uint64_t kSegMinColumns = 1u << 21;
+constexpr uint64_t kSegLongColumn = 4096;
+
+bool seg_pays(const SegForm &f, bool tail) {
+    const uint64_t R = static_cast<uint64_t>(f.C->size), total = f.outs_n * R;
+    if (total < kSegMinItems) return false;
+    if (!f.columns) return true;
+    if (R < 32) return f.V == 4 && f.splits == 1 && total >= kSegMinColumns;
+    return tail || total >= kSegMinColumns || R >= kSegLongColumn || (2 * R >= kSegLongColumn && 2 * total >= kSegMinColumns);
+}
 
 // The reduced axis is cut until the launch has about this many workgroups.
 constexpr uint64_t kSegBlocks = 2048;
@@ -1498,7 +1518,8 @@ void seg_launch(SegForm &f, int width, int64_t inner, uint64_t W) {
     f.splits = (R + f.chunk - 1) / f.chunk;
 }
 
-SegForm seg_form(const LoopB &l0, const std::set<const bh_base *> &params) {
+// (`tail`: the block is to take in a map over its outputs)
+SegForm seg_form(const LoopB &l0, const std::set<const bh_base *> &params, bool tail = false) {
     SegForm none, f;
     const uint64_t p = std::max<uint64_t>(1, jitk::parallel_ranks(l0).first);
     const std::vector<const LoopB *> chain = jitk::get_first_loop_blocks(l0);
@@ -1521,7 +1542,7 @@ SegForm seg_form(const LoopB &l0, const std::set<const bh_base *> &params) {
     if (f.C == nullptr || !f.C->isInnermost() || f.C->_sweeps.empty() || f.C->size < 16) return none;
     uint64_t outs_n = 1;
     for (uint64_t r = 0; r < p; ++r) outs_n *= static_cast<uint64_t>(std::max<int64_t>(0, chain[r]->size));
-    if (outs_n * static_cast<uint64_t>(f.C->size) < kSegMinItems || outs_n >= (1ull << 31)) return none;
+    if (outs_n >= (1ull << 31)) return none;
     std::map<const bh_base *, const bh_view *> outs;
     for (const InstrPtr &sw : f.C->_sweeps) {
         if (!bh_opcode_is_reduction(sw->opcode) || sw->sweep_axis() != f.C->rank ||
@@ -1613,7 +1634,7 @@ SegForm seg_form(const LoopB &l0, const std::set<const bh_base *> &params) {
     const uint64_t W = KernelPlan().block;
     seg_launch(f, std::max(1, std::min(4, 16 / widest)), P.size, W);
     // (a launch holds fewer than 2^32 threads, and this skeleton has a thread group for every output)
-    if (f.row_blocks * f.splits * W >= 1ull << 32) return none;
+    if (f.row_blocks * f.splits * W >= 1ull << 32 || !seg_pays(f, tail || !f.post.empty())) return none;
     return f;
 }
 
@@ -2814,7 +2835,7 @@ std::vector<LoopB> fold_row_tails(std::vector<LoopB> kernels) {
         if (a >= 0 && b >= 0) {
             const LoopB &la = out.back()._block_list[a].getLoop(), &lb = k._block_list[b].getLoop();
             if (la.rank == 0 && lb.rank == 0 && la.size == lb.size && lb.isInnermost() && lb._sweeps.empty() &&
-                seg_form(la, param_bases(out.back())).C != nullptr &&
+                seg_form(la, param_bases(out.back()), true).C != nullptr &&
                 jitk::mergeable(out.back()._block_list[a], k._block_list[b], false)) {
                 LoopB merged = out.back();
                 merged._block_list[a] = Block(jitk::merge(la, lb));

@@ -13,7 +13,8 @@ from tests.helpers import run_both
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 # (rows, cols): outputs 1 element past a thread's or workgroup's share, reduced lengths 1 past a piece
-COLUMNS = [(70001, 1 + 8), (4099, 46), (2050, 500), (129, 4096), (16, 8193), (33, 65537)]
+COLUMNS = [(70001, 1 + 8), (4099, 46), (2050, 500), (129, 4096), (16, 8193), (33, 65537),
+           (2050, 513), (1027, 2049)]
 ROWS = [(9, 70001), (46, 4099), (500, 2050), (4096, 129), (8193, 16), (65537, 33), (3, 262144 + 3)]
 
 
@@ -58,7 +59,7 @@ def test_sum_and_extremes(axis, shape, dtype):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("axis,shape", [(0, (20011, 12)), (1, (12, 20011)), (1, (5003, 40)), (0, (1024, 514))])
+@pytest.mark.parametrize("axis,shape", [(0, (20011, 12)), (1, (12, 20011)), (1, (5003, 40)), (0, (1024, 514)), (0, (2049, 514))])
 @pytest.mark.parametrize("dtype", [np.bool_, np.uint8, np.int16, np.complex64, np.complex128])
 def test_other_types(axis, shape, dtype):
     def program():
@@ -77,8 +78,20 @@ def test_other_types(axis, shape, dtype):
 
 
 @pytest.mark.gpu
+def test_few_rows_in_one_piece():
+    """17 rows of 2^21 + 4 float32: segmented without a split; whole numbers, so the sums are exact."""
+    def program():
+        x = _input((17, (1 << 21) + 4), np.int32).astype(np.float32)
+        bh.flush()
+        return [x.sum(axis=0), x.min(axis=0)]
+    got, want = run_both(program)
+    for g, w in zip(got, want):
+        np.testing.assert_array_equal(g, w)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("axis", [0, 1])
-@pytest.mark.parametrize("shape", [(3001, 64), (64, 3001), (300, 301)])
+@pytest.mark.parametrize("shape", [(3001, 64), (64, 3001), (300, 301), (4101, 66), (2050, 513), (33, 65537)])
 def test_written_and_following_work(axis, shape):
     """The loop also writes an array, the output is used after the sum, and the input is a strided, reversed or
     transposed view."""
@@ -135,6 +148,12 @@ def plan(f):
 x = bh.empty((4096, 512), np.float32)
 print(plan(lambda: x.sum(axis=0)), plan(lambda: x.sum(axis=1)), plan(lambda: x.T.sum(axis=0)))
 print(plan(lambda: x[:64, :64].sum(axis=0)), plan(lambda: x[:64, :64].sum(axis=1)))
+for dtype, shape in (("float32", (2048, 256)), ("float32", (512, 2048)), ("float32", (1023, 2049)), ("float32", (2048, 512)),
+                     ("float32", (4096, 16)), ("float32", (4095, 16)), ("float32", (32, 65536)), ("float32", (32, 65535)),
+                     ("float32", (31, 1 << 18)), ("float32", (31, 1 << 21)), ("float64", (31, 1 << 21)), ("float32", (16, 4097))):
+    y = bh.empty(shape, dtype); bh.flush()
+    print(plan(lambda: y.sum(axis=0)) + plan(lambda: y.T.sum(axis=1)))
+print(plan(lambda: x[:256, :256].mean(axis=0)), plan(lambda: x[:128, :128].mean(axis=0)), plan(lambda: x[:31].mean(axis=0)))
 bh.message("codegen: row_reduce=0")
 print(plan(lambda: x.sum(axis=1)))
 """
@@ -145,4 +164,7 @@ def test_which_reductions_are_segmented():
                        stdout=subprocess.PIPE, stderr=subprocess.STDOUT, timeout=600)
     assert r.returncode == 0, r.stdout[-3000:]
     lines = [l for l in r.stdout.splitlines() if l.startswith("[")]
-    assert lines == ["['seg'] ['seg'] ['seg']", "['row'] ['row']", "['map']"], r.stdout
+    # (columns: many rows or many elements, below 32 rows only by 16-byte loads in one launch)
+    row, seg, plain = "['row', 'row']", "['seg', 'seg']", "['map', 'map']"
+    assert lines == ["['seg'] ['seg'] ['seg']", "['row'] ['row']", row, row, row, seg, seg, row, seg, row, plain, seg, plain, plain,
+                     "['seg'] ['row', 'map'] ['map', 'map']", "['map']"], r.stdout
