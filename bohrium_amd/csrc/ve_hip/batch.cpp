@@ -407,7 +407,8 @@ void EngineHip::buildSchedule(CachedFlush &cf) {
         Level &lv = sched->levels[L];
         for (uint64_t h : hash_order[L]) {
             std::vector<PlanRef> &items = by_hash[L][h];
-            // (a segmented reduction fills the chip by itself and finalizes with a grid of its own)
+            // (a segmented reduction finalizes with a grid of its own; where many like it are faster as one batched
+            // launch they are planned as rows, crowded_reductions)
             const bool batchable =
                 cf.kernels[items[0].kernel].plans[items[0].plan].strategy != Strategy::SEG_REDUCE;
             if (batchable && items.size() >= static_cast<size_t>(batch_min)) {

@@ -1477,9 +1477,18 @@ constexpr uint64_t kSegMinItems = 1u << 16;
 constexpr uint64_t kSegMinColumns = 1u << 21;
 constexpr uint64_t kSegLongColumn = 4096;
 
-bool seg_pays(const SegForm &f, bool tail) {
+// Several of one code in one flush (`crowd`) run as one batched launch of the row skeleton, which fills the chip with
+// columns and rows that a single one leaves idle, against one or two launches each here.  60 uneven matrices, batched rows /
+// segmented, device us: by columns 300 x 320 37 / 527, 1000^2 305 / 589, 1400^2 607 / 612, 2000^2 1248 / 756, 32768 x 32 542 / 700,
+// 200000 x 8 1860 / 1027; by rows 300 x 320 12 / 375, 2000^2 289 / 514, 4000^2 1058 / 951, 20 x 50000 384 / 593,
+// 8 x 200000 1425 / 963.
+constexpr uint64_t kCrowdColumns = kSegMinColumns, kCrowdLongColumn = 1u << 15;
+constexpr uint64_t kCrowdRows = 1u << 23, kCrowdLongRow = 1u << 16;
+
+bool seg_pays(const SegForm &f, bool tail, bool crowd) {
     const uint64_t R = static_cast<uint64_t>(f.C->size), total = f.outs_n * R;
     if (total < kSegMinItems) return false;
+    if (crowd && (f.columns ? R <= kCrowdLongColumn && total < kCrowdColumns : R <= kCrowdLongRow && total < kCrowdRows)) return false;
     if (!f.columns) return true;
     if (R < 32) return f.V == 4 && f.splits == 1 && total >= kSegMinColumns;
     return tail || total >= kSegMinColumns || R >= kSegLongColumn || (2 * R >= kSegLongColumn && 2 * total >= kSegMinColumns);
@@ -1518,8 +1527,8 @@ void seg_launch(SegForm &f, int width, int64_t inner, uint64_t W) {
     f.splits = (R + f.chunk - 1) / f.chunk;
 }
 
-// (`tail`: the block is to take in a map over its outputs)
-SegForm seg_form(const LoopB &l0, const std::set<const bh_base *> &params, bool tail = false) {
+// (`tail`: the block is to take in a map over its outputs; `crowd`: see seg_pays)
+SegForm seg_form(const LoopB &l0, const std::set<const bh_base *> &params, bool crowd, bool tail = false) {
     SegForm none, f;
     const uint64_t p = std::max<uint64_t>(1, jitk::parallel_ranks(l0).first);
     const std::vector<const LoopB *> chain = jitk::get_first_loop_blocks(l0);
@@ -1634,7 +1643,7 @@ SegForm seg_form(const LoopB &l0, const std::set<const bh_base *> &params, bool 
     const uint64_t W = KernelPlan().block;
     seg_launch(f, std::max(1, std::min(4, 16 / widest)), P.size, W);
     // (a launch holds fewer than 2^32 threads, and this skeleton has a thread group for every output)
-    if (f.row_blocks * f.splits * W >= 1ull << 32 || !seg_pays(f, tail || !f.post.empty())) return none;
+    if (f.row_blocks * f.splits * W >= 1ull << 32 || !seg_pays(f, tail || !f.post.empty(), crowd)) return none;
     return f;
 }
 
@@ -1649,7 +1658,7 @@ void Writer::emit_seg_reduce() {
     const LoopB &l0 = unit._block_list.back().getLoop();
     const uint64_t p = std::max<uint64_t>(1, jitk::parallel_ranks(l0).first);
     const std::vector<const LoopB *> chain = jitk::get_first_loop_blocks(l0);
-    const SegForm f = seg_form(l0, std::set<const bh_base *>(kp.params.begin(), kp.params.end()));
+    const SegForm f = seg_form(l0, std::set<const bh_base *>(kp.params.begin(), kp.params.end()), cfg.crowd);
     if (f.C == nullptr) throw std::logic_error("seg skeleton: block has another form");
     for (const bh_instruction *i : f.seeds) skip.insert(i);
     const LoopB &C = *f.C;
@@ -2826,29 +2835,61 @@ int only_loop(const LoopB &kernel) {
 }
 } // namespace
 
-std::vector<LoopB> fold_row_tails(std::vector<LoopB> kernels) {
+std::vector<bool> crowded_reductions(const std::vector<LoopB> &kernels, int batch_min) {
+    std::vector<bool> out(kernels.size(), false);
+    if (batch_min <= 0 || kernels.size() < static_cast<size_t>(batch_min)) return out;
+    // Segmented blocks that a crowd leaves to the rows, by what their code is made of: operations, types, axis.
+    std::map<std::string, std::vector<size_t> > like;
+    for (size_t k = 0; k < kernels.size(); ++k) {
+        const std::set<const bh_base *> params = param_bases(kernels[k]);
+        std::string key;
+        for (const Block &b : kernels[k]._block_list) {
+            if (b.isInstr() || b.getLoop().rank != 0) continue;
+            const SegForm f = seg_form(b.getLoop(), params, false, true);
+            if (f.C == nullptr || seg_form(b.getLoop(), params, true, true).C != nullptr) continue;
+            key += f.columns ? "c" : "r";
+            for (const InstrPtr &i : jitk::allInstr(*f.C)) {
+                if (bh_opcode_is_system(i->opcode)) continue;
+                key += std::to_string(i->opcode) + ":";
+                for (const bh_view &v : i->operand) key += v.isConstant() ? "-" : std::to_string(static_cast<int>(v.base->dtype())) + "/" + std::to_string(v.ndim) + ",";
+            }
+        }
+        if (!key.empty()) like[key].push_back(k);
+    }
+    for (const auto &l : like)
+        if (l.second.size() >= static_cast<size_t>(batch_min))
+            for (size_t k : l.second) out[k] = true;
+    return out;
+}
+
+std::vector<LoopB> fold_row_tails(std::vector<LoopB> kernels, int batch_min) {
+    const std::vector<bool> crowd = crowded_reductions(kernels, batch_min);
     std::vector<LoopB> out;
-    for (LoopB &k : kernels) {
+    bool crowd_a = false;  // of out.back()
+    for (size_t n = 0; n < kernels.size(); ++n) {
+        LoopB &k = kernels[n];
         const int b = only_loop(k);
-        const int a = out.empty() ? -1 : only_loop(out.back());
+        const int a = out.empty() || crowd_a ? -1 : only_loop(out.back());
         bool folded = false;
         if (a >= 0 && b >= 0) {
             const LoopB &la = out.back()._block_list[a].getLoop(), &lb = k._block_list[b].getLoop();
             if (la.rank == 0 && lb.rank == 0 && la.size == lb.size && lb.isInnermost() && lb._sweeps.empty() &&
-                seg_form(la, param_bases(out.back()), true).C != nullptr &&
+                seg_form(la, param_bases(out.back()), false, true).C != nullptr &&
                 jitk::mergeable(out.back()._block_list[a], k._block_list[b], false)) {
                 LoopB merged = out.back();
                 merged._block_list[a] = Block(jitk::merge(la, lb));
                 for (size_t i = 0; i < k._block_list.size(); ++i)
                     if (static_cast<int>(i) != b) merged._block_list.push_back(k._block_list[i]);
                 merged.metadataUpdate();
-                if (seg_form(merged._block_list[a].getLoop(), param_bases(merged)).C != nullptr) {
+                if (seg_form(merged._block_list[a].getLoop(), param_bases(merged), false).C != nullptr) {
                     out.back() = std::move(merged);
                     folded = true;
                 }
             }
         }
-        if (!folded) out.push_back(std::move(k));
+        if (folded) continue;
+        out.push_back(std::move(k));
+        crowd_a = crowd[n];
     }
     return out;
 }
@@ -2953,7 +2994,7 @@ std::vector<KernelPlan> plan_kernel(const LoopB &kernel, const WriterConfig &cfg
         unit._block_list.push_back(b);
         if (s == Strategy::MAP && cfg.row_reduce) {
             unit.metadataUpdate();
-            if (seg_form(l0, param_bases(unit)).C != nullptr) {
+            if (seg_form(l0, param_bases(unit), cfg.crowd).C != nullptr) {
                 s = Strategy::SEG_REDUCE;
             } else if (!row_lane_loops(l0).empty()) {
                 s = Strategy::ROW_REDUCE;

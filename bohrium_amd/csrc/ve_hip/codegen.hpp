@@ -14,7 +14,7 @@
  *                loop (row sums of an expression): one wave per row, lanes stride the
  *                row (coalesced), wave64 butterfly, lane 0 stores.
  *   SEG_REDUCE   one reduction loop per element of the parallel ranks (a sum over one axis of a
- *                matrix) when the matrix is large: wide coalesced loads along whichever axis is
+ *                matrix) when the matrix is large, or larger than that where many share a flush: wide coalesced loads along whichever axis is
  *                contiguous, and the reduced axis split over workgroups (partials folded by a
  *                finalize kernel) when the outputs alone do not fill the chip.
  *   SERIAL       anything else, executed by one thread (always correct).
@@ -117,6 +117,7 @@ struct WriterConfig {
      * in 8 contiguous parts, one per XCD (workgroup b runs on XCD b mod 8): a row's neighbours are
      * read under the same L2. */
     bool xcd_parts = true;
+    bool crowd = false;      // the kernel being planned is one of many like it in its flush (crowded_reductions)
     uint32_t epoch = 1;      // look-back flag generation (changes every launch)
 };
 
@@ -127,7 +128,11 @@ std::vector<jitk::LoopB> fold_serial_tails(std::vector<jitk::LoopB> kernels);
 /* Append each map over the outputs of the segmented reduction before it (the division of a column mean) to that
  * reduction's loop: it then runs with the finalized outputs, in their registers.  (The fuser has no chance
  * to: the loops have one shape only after the reduction was pushed inwards.) */
-std::vector<jitk::LoopB> fold_row_tails(std::vector<jitk::LoopB> kernels);
+std::vector<jitk::LoopB> fold_row_tails(std::vector<jitk::LoopB> kernels, int batch_min);
+
+/* Which kernels hold one of at least batch_min like segmented reductions that a batched launch of rows runs faster
+ * (WriterConfig::crowd). */
+std::vector<bool> crowded_reductions(const std::vector<jitk::LoopB> &kernels, int batch_min);
 
 /* Check that every operand dimension is iterated within its extent by the loop of the matching
  * rank (what the generated indexing assumes); returns "" or a description of each violation. */

@@ -861,7 +861,8 @@ void EngineHip::handleExecution(BhIR *bhir) {
         ++flush_cache_misses;
         std::unordered_map<const bh_base *, int> base2ord;  // the flush's base ordinals (inverse of ord2base)
         for (size_t o = 0; o < ord2base.size(); ++o) base2ord.emplace(ord2base[o], static_cast<int>(o));
-        std::vector<jitk::LoopB> kernels = fold_row_tails(fold_serial_tails(jitk::get_kernel_list(instr_list, fusion_config)));
+        std::vector<jitk::LoopB> kernels = fold_row_tails(fold_serial_tails(jitk::get_kernel_list(instr_list, fusion_config)), batch_min);
+        const std::vector<bool> crowd = crowded_reductions(kernels, batch_min);
         // A kernel releases the bases freed in it when it ends: no later kernel may use them.
         {
             std::set<const bh_base *> released;
@@ -876,7 +877,9 @@ void EngineHip::handleExecution(BhIR *bhir) {
         stats.time_fuse += seconds_since(t);
         t = std::chrono::steady_clock::now();
         CachedFlush cf;
-        for (const jitk::LoopB &kernel : kernels) {
+        for (size_t k = 0; k < kernels.size(); ++k) {
+            const jitk::LoopB &kernel = kernels[k];
+            wcfg.crowd = crowd[k];
             if (debug) std::fprintf(stderr, "[hip] kernel:\n%s", kernel.pprint().c_str());
             CachedKernel ck;
             if (!kernel.isSystemOnly()) {
