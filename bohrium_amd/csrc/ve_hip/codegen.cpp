@@ -398,17 +398,22 @@ struct TiledForm {
     int side = 0;    // T
 };
 
-// Below this many elements (a few hundred KB, held by the L2s) one round of latency bounds the map either way.
-constexpr uint64_t kTileMinItems = 1u << 16;
+// Tiled from 2^20 elements on, or where a transposed view has 6 MB, half as much again as one XCD's L2: below, the L2s
+// hold the lines of the flat walk until their other elements are asked for, and a tile is two rounds of latency for one.
+// Flat / tiled, device us: x + x.T float32 512^2 6.3 / 6.2, 724^2 6.8 / 9.4, 860^2 7.8 / 9.6, 1024^2 8.7 / 6.6, x + y.T 1300^2
+// 15.2 / 12.8; four maps of which two are tiled float64 760^2 28.4 / 31.2, 960^2 36.3 / 29.1; x.T * 1.5 and x + x.T together
+// complex128 512^2 13.2 / 14.1, 860^2 26.2 / 17.6.
+constexpr uint64_t kTileMinItems = 1u << 20;
+constexpr int64_t kTileMinBytes = 6 << 20;
 
 TiledForm tiled_form(const std::vector<const LoopB *> &chain, uint64_t p, const std::vector<const bh_view *> &reads) {
     TiledForm f;
     if (p < 2) return f;
     uint64_t total = 1;
     for (uint64_t r = 0; r < p; ++r) total *= static_cast<uint64_t>(std::max<int64_t>(0, chain[r]->size));
-    if (total < kTileMinItems) return f;
     const int64_t a = static_cast<int64_t>(p) - 1;
-    int bytes = 0, widest = 1;
+    int bytes = 0;
+    int64_t largest = 0;
     for (const bh_view *v : reads) {
         if (v->ndim <= a || v->hasSlide()) continue;
         if (v->stride[a] == 0 || std::abs(v->stride[a]) < 8) continue;
@@ -420,8 +425,9 @@ TiledForm tiled_form(const std::vector<const LoopB *> &chain, uint64_t p, const 
         f.views.push_back(v);
         const int sz = bh_type_size(v->base->dtype());
         bytes += sz;
-        widest = std::max(widest, sz);
+        largest = std::max(largest, reached_bytes(*v));
     }
+    if (total < kTileMinItems && largest < kTileMinBytes) return TiledForm();
     if (f.views.empty() || chain[a]->size < 32 || chain[f.q]->size < 32) return TiledForm();
     f.side = 65 * 64 * bytes <= 40960 ? 64 : 32;
     while (33 * 32 * bytes > 65536) {
