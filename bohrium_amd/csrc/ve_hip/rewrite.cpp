@@ -329,7 +329,7 @@ int recompute_temporaries(std::vector<bh_instruction *> &list, RewriteStore &sto
                         if (list[j]->opcode == BH_FREE) {
                             if (list[j]->operand[0].base != v.base) continue;
                             same &= distinct_elements(v) * 8 <= T->nelem();
-                            late.push_back(j);
+                            if (std::find(late.begin(), late.end(), j) == late.end()) late.push_back(j);  // (v + v.T)
                         } else {
                             same &= !writes(list[j], v.base);
                         }

@@ -104,3 +104,18 @@ for count in (1200, 300):
                        stdout=subprocess.PIPE, stderr=subprocess.STDOUT, timeout=600)
     assert r.returncode == 0, r.stdout[-3000:]
     assert r.stdout.split() == ["0", "1"], r.stdout
+
+
+def test_a_freed_input_named_twice_is_freed_once(tmp_path):
+    """c = v[:, None] + v[None, :] is repeated behind the free of v: the free moves behind the reader, once."""
+    lib, csrc = os.path.join(ROOT, "bohrium_amd", "lib"), os.path.join(ROOT, "bohrium_amd", "csrc")
+    exe = str(tmp_path / "recompute_check")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-I" + os.path.join(csrc, "include"), "-I" + csrc,
+                    os.path.join(ROOT, "tests", "csrc", "recompute_check.cpp"), os.path.join(csrc, "ve_hip", "rewrite.cpp"),
+                    "-o", exe, "-L" + lib, "-lbh", "-Wl,-rpath," + lib], check=True)
+    out = subprocess.run([exe], stdout=subprocess.PIPE, text=True, check=True, timeout=60).stdout.splitlines()
+    assert out[0] == "rewritten 1", out
+    assert out.count("BH_FREE v") == 1, out
+    at = [k for k, l in enumerate(out) if l.startswith("BH_DIVIDE z again")]
+    assert len(at) == 1 and out[at[0] - 1] == "BH_ADD again v v" and out.index("BH_FREE v") > at[0], out
+    assert len(out) == len(set(out)), out
