@@ -123,10 +123,20 @@ struct Tile {
             int r, k;
             chunk(e, r, k);
             const int64_t gr = source(r0, r, R);
-            const T *q = KCONT ? P + gr * ld + k : P + k * ld + gr;
+            p[e] = KCONT ? P + gr * ld + k : P + k * ld + gr;
+        }
+        // A whole step by 16-byte loads, like the others (element by element 2048 x 2048 x 64 float32 took 11.1 us, 9.8 so).
+        if (kn == kBK) {
+            next();
+            return;
+        }
 #pragma unroll
-            for (int j = 0; j < V; ++j) reg[e * V + j] = (KCONT ? k + j : k) < kn ? q[j] : T(0);
-            p[e] = q + (KCONT ? kn : kn * ld);
+        for (int e = 0; e < CH; ++e) {
+            int r, k;
+            chunk(e, r, k);
+#pragma unroll
+            for (int j = 0; j < V; ++j) reg[e * V + j] = (KCONT ? k + j : k) < kn ? p[e][j] : T(0);
+            p[e] += KCONT ? kn : kn * ld;
         }
     }
     __device__ __forceinline__ void next() {

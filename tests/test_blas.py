@@ -392,3 +392,18 @@ def test_gemm_infinities_stay_in_their_row_and_column():
         assert np.isinf(c[n // 2, :-1]).all() and np.isnan(c[:, -1]).all()
         c[n // 2] = 37
         np.testing.assert_array_equal(c[:, :-1], np.full((n, n - 1), 37.0))
+
+
+# K of one step, two and one more, whole steps and remainders, on tiles (1100 x 1030) ...
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.complex128, np.complex64])
+@pytest.mark.parametrize("k", [1, 15, 16, 17, 32, 33, 48])
+def test_gemm_short_k(dtype, k):
+    import bohrium_amd as bh
+    for m, n in [(1100, 1030)] + SHORT:
+        a, b = _rand((m, k), dtype, 1), _rand((k, n), dtype, 2)
+        _check(bh.blas.gemm(bh.array(a), bh.array(b)).asnumpy(), a, b, dtype)
+        _check(bh.blas.gemmt(bh.array(np.ascontiguousarray(a.T)), bh.array(b)).asnumpy(), a, b, dtype)
+
+
+SHORT = []
