@@ -679,9 +679,15 @@ void launch_slice_tile(const Gemm &g) {
 
 template <typename E, bool TA, bool TB, bool CONJB, bool UPPER, bool REALDIAG, bool SCALED>
 void launch_slice(const Gemm &g) {
-    if (tiles(g, 32, 32) >= kFill)
+    // One or two steps of K: further waves would only wait for the fold (8 x 30000 x 16 c128 17.9 us with a 32 x 32 tile of
+    // 4 waves, 4.4 so; 900 x 900 x 16 f64 6.6 -> 4.6).  16 rows or columns at most: a tile of 32 is at least half padding, and
+    // complex products are bound by its MFMAs (15 x 20000 x 200 c128 37.5 us, 20.4 with the small tile).
+    constexpr bool complex = sizeof(E) != sizeof(typename Prod<E>::Real);
+    if (g.k <= 32)
+        launch_slice_tile<E, TA, TB, CONJB, UPPER, REALDIAG, SCALED, 1, 1, 2>(g);
+    else if (tiles(g, 32, 32) >= kFill && !(complex && std::min(g.m, g.n) <= 16))
         launch_slice_tile<E, TA, TB, CONJB, UPPER, REALDIAG, SCALED, 2, 2, 4>(g);
-    else if (sizeof(E) == sizeof(typename Prod<E>::Real) && tiles(g, 16, 32) >= kFill)
+    else if (!complex && tiles(g, 16, 32) >= kFill)
         launch_slice_tile<E, TA, TB, CONJB, UPPER, REALDIAG, SCALED, 1, 2, 8>(g);
     else
         launch_slice_tile<E, TA, TB, CONJB, UPPER, REALDIAG, SCALED, 1, 1, 8>(g);

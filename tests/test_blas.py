@@ -406,4 +406,6 @@ def test_gemm_short_k(dtype, k):
         _check(bh.blas.gemmt(bh.array(np.ascontiguousarray(a.T)), bh.array(b)).asnumpy(), a, b, dtype)
 
 
-SHORT = []
+# ... and on tiles of 16 x 16 by two waves, which these are too small or too thin for 64 x 64 tiles with (K up to 32; by
+# eight waves from there on where a complex product has at most 16 rows or columns)
+SHORT = [(8, 5000), (5000, 8), (16, 9001), (9001, 15), (17, 9000), (9000, 17), (900, 870), (1, 1)]
