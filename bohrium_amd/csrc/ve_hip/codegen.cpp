@@ -1466,6 +1466,7 @@ struct SegForm {
      * workgroups cover the outputs, times `splits` pieces of `chunk` elements of the reduced axis. */
     int V = 1, U = 4;
     uint64_t outs_n = 1, lanes = 1, row_blocks = 1, splits = 1, chunk = 1, w = 1;
+    uint64_t reads = 0;  // views that C reads an element of per iteration (broadcasts along either axis left out)
 };
 
 // Where one reduction is segmented, from device times of sums of x * x in float32 and float64 (one launch and its gap
@@ -1474,7 +1475,8 @@ struct SegForm {
 // 8192: row 16.6, seg 6.1 us; 131072 x 16: map 8.0, seg 6.3).
 // Columns are split and finalized, so the row skeleton's single launch wins while its waves' walks down the columns
 // are short and their lines stay in the L2s: row / seg 2048 x 256 8.6 / 9.4 us, 512 x 2048 6.7 / 9.4, 1024 x 1500 11.1 / 8.8
-// (host and device together 11.5 / 14.6); 4096 x 16 11.7 / 8.2, 2048 x 700 16.1 / 9.0, 40 x 60000 15.8 / 9.7.
+// (host and device together 11.5 / 14.6); 4096 x 16 11.7 / 8.2, 2048 x 700 16.1 / 9.0, 40 x 60000 15.8 / 9.7.  Its time goes
+// with the loads: sums over three arrays 512^2 7.3 / 8.9, 900^2 15.6 / 10.3, 750 x 1500 21.9 / 10.4.
 // Fewer than 32 rows: a thread per column reads them coalesced in one launch.  map / seg 16 x 2^20 float32 14.7 / 40.3, 31 x 2^18
 // 8.3 / 17.4; 16-byte loads without a split are ahead: 16 x 2^22 64 / 51, 31 x 2^21 56 / 47.
 // With a map over the outputs in its finalize (a mean) this skeleton has no launch more: x - x.mean(0) of 256^2 18.5 / 15.3
@@ -1492,12 +1494,12 @@ constexpr uint64_t kCrowdColumns = kSegMinColumns, kCrowdLongColumn = 1u << 15;
 constexpr uint64_t kCrowdRows = 1u << 23, kCrowdLongRow = 1u << 16;
 
 bool seg_pays(const SegForm &f, bool tail, bool crowd) {
-    const uint64_t R = static_cast<uint64_t>(f.C->size), total = f.outs_n * R;
+    const uint64_t R = static_cast<uint64_t>(f.C->size), total = f.outs_n * R, loads = total * std::max<uint64_t>(1, f.reads);
     if (total < kSegMinItems) return false;
-    if (crowd && (f.columns ? R <= kCrowdLongColumn && total < kCrowdColumns : R <= kCrowdLongRow && total < kCrowdRows)) return false;
+    if (crowd && (f.columns ? R <= kCrowdLongColumn && loads < kCrowdColumns : R <= kCrowdLongRow && loads < kCrowdRows)) return false;
     if (!f.columns) return true;
-    if (R < 32) return f.V == 4 && f.splits == 1 && total >= kSegMinColumns;
-    return tail || total >= kSegMinColumns || R >= kSegLongColumn || (2 * R >= kSegLongColumn && 2 * total >= kSegMinColumns);
+    if (R < 32) return f.V == 4 && f.splits == 1;
+    return tail || loads >= kSegMinColumns || R >= kSegLongColumn || (2 * R >= kSegLongColumn && 2 * loads >= kSegMinColumns);
 }
 
 // The reduced axis is cut until the launch has about this many workgroups.
@@ -1634,6 +1636,7 @@ SegForm seg_form(const LoopB &l0, const std::set<const bh_base *> &params, bool 
             const bh_view &v = i->operand[o];
             if (v.isConstant() || !params.count(v.base) || v.ndim <= c || !seen.insert(vkey(v)).second) continue;
             if (v.stride[c] == 0 || v.stride[a] == 0) continue;  // (broadcast: a fraction of the elements)
+            ++f.reads;
             const int sz = bh_type_size(v.base->dtype());
             if (v.stride[c] == 1 && v.shape[c] > 1 && v.stride[a] != 1) {
                 rows += sz;

@@ -172,6 +172,9 @@ for dtype, shape in (("float32", (2048, 256)), ("float32", (512, 2048)), ("float
                      ("float32", (31, 1 << 18)), ("float32", (31, 1 << 21)), ("float64", (31, 1 << 21)), ("float32", (16, 4097))):
     y = bh.empty(shape, dtype); bh.flush()
     print(plan(lambda: y.sum(axis=0)) + plan(lambda: y.T.sum(axis=1)))
+y, z = bh.empty((4096, 512), np.float32), bh.empty((4096, 512), np.float32); bh.flush()
+for r in (1360, 1366, 1400):  # three arrays: 2^21 loads are 1365.3 rows
+    print(plan(lambda: (x[:r] * y[:r] + z[:r]).sum(axis=0)) + plan(lambda: (x[:r] * 2 + x[:r]).sum(axis=0)))
 print(plan(lambda: x[:256, :256].mean(axis=0)), plan(lambda: x[:128, :128].mean(axis=0)), plan(lambda: x[:31].mean(axis=0)))
 bh.message("codegen: row_reduce=0")
 print(plan(lambda: x.sum(axis=1)))
@@ -186,4 +189,4 @@ def test_which_reductions_are_segmented():
     # (columns: many rows or many elements, below 32 rows only by 16-byte loads in one launch)
     row, seg, plain = "['row', 'row']", "['seg', 'seg']", "['map', 'map']"
     assert lines == ["['seg'] ['seg'] ['seg']", "['row'] ['row']", row, row, row, seg, seg, row, seg, row, plain, seg, plain, plain,
-                     "['seg'] ['row', 'map'] ['map', 'map']", "['map']"], r.stdout
+                     row, "['seg', 'row']", "['seg', 'row']", "['seg'] ['row', 'map'] ['map', 'map']", "['map']"], r.stdout
