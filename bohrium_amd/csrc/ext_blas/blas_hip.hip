@@ -178,9 +178,9 @@ struct Tile {
 // The LDS tiles are double-buffered: while the matrix cores work on one K step, the next one is
 // loaded into registers and then stored into the other buffer; one barrier per K step.  Two waves a SIMD: the
 // epilogue alone would take the f64 128 x 128 kernel to 278 registers and one wave.
-// Bound by the MFMA rate (counters: the matrix cores were busy 76 % of the cycles while the loads waited at
-// bounds checks).  Measured with the checks out of the loop: 4096^3 f64 2364 -> 2078 us (66.1 TFLOP/s; the
-// library 66-69), f32 1118 -> 1029 us; 2000 x 1500 x 2500 f64 344 -> 267 us, f32 189 -> 155 us.
+// Bound by the MFMA rate (counters: the matrix cores are busy 83 % of the cycles of the f64 128 x 128 kernel).
+// Measured against loads that wait at bounds checks in the loop: 4096^3 f64 2363 -> 2072 us (66.3 TFLOP/s; the library
+// 67-69), f32 1120 -> 1017 us; 2000 x 1500 x 2500 f64 344 -> 269 us, f32 189 -> 144 us.
 template <typename T, bool TA, bool TB, bool UPPER, int TM, int TN, int BK, bool SCALED>
 __global__ void __launch_bounds__(kThreads, 2)
 gemm_mfma(const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C, int64_t M, int64_t N, int64_t K,
@@ -291,8 +291,8 @@ template <typename R> __device__ __forceinline__ Cplx<R> msub(Cplx<R> s, Cplx<R>
 // TM TN BK MFMAs of 64 (f64) or 32 (f32) cycles for (TM + TN) BK / 4 LDS reads.  Tiles, staging and double
 // buffering as in gemm_mfma; the LDS rows are padded to an odd number of 16-byte elements (c128) or to two
 // 8-byte elements more than a multiple of 16 (c64), so the 16-lane groups of a read fall in disjoint banks.
-// Measured against one FMA thread per element of C: 4096^3 c128 22.8 -> 65.2 TFLOP/s (24.1 -> 8.4 ms), c64
-// 34.6 -> 121 TFLOP/s; 2000 x 1500 x 2500 c128 2678 -> 984 us, with the bounds checks out of the loop 901 us.
+// Measured against one FMA thread per element of C: 4096^3 c128 24.4 -> 7.74 ms (22.5 -> 71.0 TFLOP/s), c64
+// 34.5 -> 131.8 TFLOP/s; 2000 x 1500 x 2500 c128 2771 -> 920 us.  The matrix cores are busy 86 % of the cycles (c128).
 template <typename R, bool KCONT, int ROWS, int kBK>
 struct CTile {
     static constexpr int CH = ROWS * kBK / kThreads;
@@ -442,8 +442,8 @@ gemm_complex(const Cplx<R> *__restrict__ A, const Cplx<R> *__restrict__ B, Cplx<
 // K.  Here a workgroup computes a 16 TM x 16 TN tile with WAVES waves, wave w the K steps w, w + WAVES, ...
 // of 16, straight from global memory (no sharing to stage for; a lane loads 4 neighbouring k where K is
 // contiguous), and the partial tiles are folded through LDS in a fixed order.  Measured: 100 x 100 x 4000 f64
-// 323 -> 24 us, f32 204 -> 12, c128 292 -> 43; 512^3 f64 30 -> 11; 256^3 f64 16 -> 4.4, c128 14.4 -> 6.4;
-// 2048 x 64 x 2048 f32 67 -> 13 us.
+// 323 -> 24 us, f32 204 -> 11, c128 292 -> 43; 512^3 f64 30 -> 9.4; 256^3 f64 16 -> 4.1, c128 14.6 -> 5.6;
+// 2048 x 64 x 2048 f32 67 -> 11.4 us.
 template <typename E> struct Prod {
     typedef typename Mfma<E>::Acc Acc;
     typedef E Real;
@@ -661,8 +661,9 @@ int64_t tiles(const Gemm &g, int64_t bm, int64_t bn) { return ((g.m + bm - 1) / 
 
 // The 256 CUs need a workgroup each: fewer 64 x 64 tiles than that, and K is split over waves instead
 // (gemm_slice), with the largest tile that still gives 256 workgroups.  Measured, tile / slice: 1001 x 777 x
-// 1303 (208 tiles) f64 69 / 63 us, f32 75 / 40, c128 188 / 205, c64 122 / 105; 512^3 (64 tiles) f64 26 / 11,
-// f32 18 / 7, c128 74 / 26, c64 47 / 15; 2000 x 1500 x 2500 (768 tiles) f64 267 / 352, f32 155 / 209.
+// 1303 (208 tiles) f64 66 / 60 us, f32 40 / 38, c128 186 / 201, c64 113 / 99; 512^3 (64 tiles) f64 25 / 9.4,
+// f32 15 / 6.1, c128 73 / 24, c64 46 / 13; 1024^3 (256 tiles) f64 49 / 51, f32 30 / 29, c128 148 / 157, c64 90 / 78; 2000 x
+// 1500 x 2500 (768 tiles) f64 269 / 349, f32 144 / 210, c128 919 / 1101, c64 510 / 540.
 // (The tiles' chunks need as many rows and columns as a vector has elements.)
 constexpr int64_t kFill = 256;
 bool use_tiles(const Gemm &g) { return tiles(g, 64, 64) >= kFill && g.m >= 16 && g.n >= 16; }

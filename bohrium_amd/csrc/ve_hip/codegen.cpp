@@ -390,8 +390,8 @@ struct KernelParam {
 // a cache line for 64 elements, bound by the L2 request rate.  Here a workgroup takes a T x T tile of
 // the two axes, copies the transposed views' tile through LDS with its lanes along their contiguous
 // axis, and computes with its lanes along the innermost axis (a row of T + 1 elements in LDS, so
-// neither direction conflicts).  Measured on 4096^2 float32: a.T * 1 64.4 -> 30.7 us (4.4 TB/s),
-// (a + a.T) * 0.5 70.1 -> 39.0 us.
+// neither direction conflicts).  Measured on 4096^2 float32: a.T * 1 64.4 -> 29.0 us (4.6 TB/s),
+// (a + a.T) * 0.5 70.1 -> 36.8 us.
 struct TiledForm {
     int64_t q = -1;  // the axis along which the transposed views are contiguous
     std::vector<const bh_view *> views;
@@ -995,8 +995,8 @@ bool shifted_reads(const LoopB &l) {
 // copy rate).  Here a thread owns V neighbouring columns and walks down a band of rows with a window of the
 // array in registers: every element of the band is loaded once per thread (16-byte loads of the V columns
 // plus the side columns), and a group of `ur` rows is loaded before it is computed.  Measured on the 8192^2
-// float32 5-point sweep with max|new - old|: 133 -> 106 us (4.0 -> 5.1 TB/s; a plain copy reaches 5.6), 200 sweeps
-// 27.3 -> 21.9 ms.
+// float32 5-point sweep with max|new - old|: 134 -> 103 us (4.0 -> 5.2 TB/s; a plain copy reaches 5.6), 200 sweeps
+// 27.3 -> 21.3 ms (23.9 of them without the stores past the caches, kStreamBytes).
 namespace {
 // A window: the views of one base with equal strides, as offsets (row, column) from the first.
 struct Window {
@@ -1034,7 +1034,9 @@ std::vector<Window> stencil_windows(const std::vector<const bh_view *> &reads) {
 }
 
 // Fewer elements than this (2^20: 1024^2, 256 workgroups of single row groups) leave too few bands to fill the chip,
-// and their arrays stay in the L2s, where the element walk's repeated loads are cheap.
+// and their arrays stay in the L2s, where the element walk's repeated loads are cheap.  Element walk / this, device us of
+// the 5-point sum: float32 512^2 6.3 / 6.2, 1024^2 6.9 / 6.6, 1500^2 8.3 / 8.1, 4096^2 28.2 / 23.7; float64 512^2 6.4 / 6.4,
+// 1024^2 8.5 / 7.0, 1500^2 12.2 / 9.8, 4096^2 61 / 45.
 constexpr int64_t kStencilMinItems = 1 << 20;
 } // namespace
 
@@ -1660,9 +1662,9 @@ SegForm seg_form(const LoopB &l0, const std::set<const bh_base *> &params, bool 
 // Bound by HBM when the whole chip loads.  What the row skeleton left idle: a column sum ran one wave
 // per column with its lanes a row apart (one 64-byte request per lane and element), and few outputs
 // gave few waves.  Here lanes always run along the contiguous axis with 16-byte loads, and the reduced
-// axis is cut into `splits` pieces until the launch has about kSegBlocks workgroups.  Measured on float32:
-// mean, variance and standardised matrix of 100000 x 500 by columns 1792 -> 231 us (the two reduction
-// kernels 0.81 and 0.88 ms before), of 16384 x 3000 by rows 223 -> 198 us (4-byte loads before).
+// axis is cut into `splits` pieces until the launch has about kSegBlocks workgroups.  Measured on float32
+// sums: 100000 x 500 by columns 536 -> 40 us (5.0 TB/s), 65536 x 16 137 -> 8.6; by rows (4-byte loads before) 512 x 4096
+// 10.6 -> 6.0 us, 64 x 16384 29 -> 8.3.
 void Writer::emit_seg_reduce() {
     const LoopB &l0 = unit._block_list.back().getLoop();
     const uint64_t p = std::max<uint64_t>(1, jitk::parallel_ranks(l0).first);
@@ -2485,7 +2487,8 @@ void Writer::emit_scan() {
     // contiguous, and one wave scan per run instead of one per element.  The elements first (every load of
     // the tile issued before the first wave scan waits for one): a full tile without bounds checks, the
     // last tile with them; both unrolled, so that v_ stays in registers.  Measured: the int64 running count of
-    // 6e7 float32 276 -> 195 us (one element per thread and wave scan, 16 per tile and thread, before; 64 now).
+    // 6e7 float32 279 -> 180 us of device time (one element per thread and wave scan, 16 per tile and thread, before; 64
+    // now).  At no tile size and length is it behind the form before: 8 per thread 391 -> 385 us, 1e6 elements 17.8 -> 17.2.
     for (int full = 1; full >= 0; --full) {
         if (full)
             body << "  if (tb_ + " << tile_elems << " <= n" << lid.at(&l0) << ") {\n";

@@ -44,8 +44,8 @@ int unflatten_full_reductions(std::vector<bh_instruction *> &list, RewriteStore 
  * read of its input.  The same operation on the same values: results do not change.  Conditions: the
  * temporary is freed in the flush, not synced, written once and read through its whole view; its
  * inputs are not written between (a small one freed between lives until the later reader).
- * Measured with the maps folded into the reductions before them (fold_row_tails): column statistics and the
- * standardised matrix of 100000 x 500 float32 231 -> 176 us, row statistics of 16384 x 3000 198 -> 155 us.
+ * Measured: mean, variance and standardised matrix of 100000 x 500 float32 by columns 195 -> 157 us of device time, of
+ * 16384 x 3000 by rows 173 -> 137 us.
  * Lists of more than 4096 instructions are left alone: with 4096 uneven arrays in one flush (37,000 instructions, the
  * running counts' casts all candidates) the search took 100 ms of a flush of 50.
  * Returns the number of readers rewritten. */
